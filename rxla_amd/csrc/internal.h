@@ -160,6 +160,8 @@ int noalloc_device_setup(int device, hipStream_t stream);
 int rt_alloc(Runtime *rt, size_t bytes, void **out);
 void rt_free(Runtime *rt, void *ptr, size_t bytes);
 int ensure_workspace(Runtime *rt, Workspace &ws, size_t bytes, bool zero);
+// Whether the runtime's stream is being captured into a graph
+bool stream_capturing(const Runtime *rt);
 // Validates a buffer shape (known dtype, rank <= RXW8_MAX_RANK, dims >= 0,
 // element count and byte size within int64 by checked products) and returns
 // its byte size; INVALID_ARGUMENT otherwise. Every buffer is created through

@@ -1416,7 +1416,9 @@ rxw8_gqa_prefill_r2_d128_g8(PrefillArgs a) {
 }
 
 // ---- generic decode attention (any D <= 256, any group, f32 or bf16 cache):
-// one workgroup per (b, query head); scores staged in LDS (Lmax <= 8192).
+// one workgroup per (b, query head); scores staged in LDS (Lmax <= 8192). Head
+// widths 64, 128 and 256 run on the f32 matrix-core kernels instead
+// (attention_f32.hip); this one takes the other widths and unaligned operands.
 struct AttnGenericArgs {
   const void *q;
   const void *kc;
@@ -1503,6 +1505,9 @@ extern "C" __global__ void __launch_bounds__(256) rxw8_gqa_decode_generic(AttnGe
 // sees keys 0 .. st + i only, st = clamp(starts[b], 0, Sk - Sq) (the
 // reference's causal mask key_pos <= q_pos for rows at positions st + i;
 // the keys past it are skipped, which adds exactly nothing to the softmax).
+//
+// Head widths 64, 128 and 256 (K and V alike) run on the f32 matrix-core tiles
+// (attention_f32.hip); this kernel takes every other shape.
 //
 // One wave per output row (b, h, i). The row's q sits in the wave's LDS
 // slice; keys go in chunks of 64 (lane = key: a sequential f32 dot product

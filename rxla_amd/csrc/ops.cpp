@@ -136,6 +136,25 @@ struct GqaGeneralArgs {
   const int32_t *starts;
 };
 
+struct GqaTileArgs {
+  const void *q, *k, *v;
+  const float *mask;
+  void *out;
+  int64_t bdim[4];
+  int64_t mb[4];
+  int64_t msh, msi, msj;
+  int64_t q_sb, q_sh, q_si;
+  int64_t o_sb, o_sh, o_si;
+  int64_t k_sb, k_sh;
+  int64_t v_sb, v_sh;
+  const int32_t *starts, *lens, *slots;
+  float *part;
+  int *counters;
+  int NB, Hq, Hkv, Sq, Sk, tiles, nsplit;
+  float scale;
+  int q_bf16, out_bf16;
+};
+
 struct CausalMaskArgs {
   const int32_t *qpos, *kpos;
   float *out;
@@ -1038,6 +1057,109 @@ int bf16_linear_launch(Runtime *rt, const void *x, int x_f32, const uint16_t *w,
   return run_generic_linear(rt, x, x_f32, w, 1, nullptr, y, y_f32, M, N, K, K, 1);
 }
 
+// Split partials and counters of one f32 attention launch at most: what the
+// no-allocation entry's fixed array holds, so that both entries run one plan.
+constexpr size_t kF32PartialMax = RXW8_NOALLOC_PARTIAL_BYTES;
+constexpr int64_t kF32UnitsMax = RXW8_NOALLOC_COUNTER_BYTES / sizeof(int);
+
+// Attention on the f32 matrix-core kernels (kernels/attention_f32.hip) for
+// head widths 64 / 128 / 256 (K and V alike), 16-byte aligned operands and
+// K/V planes within 32-bit byte offsets; else UNIMPLEMENTED (nothing
+// launched) and the caller's scalar kernel takes the call. `a` carries
+// everything but the plan.
+//   Up to 8 rows (query heads of a kv head x queries; decode steps): the quad
+// kernel, whose 8 waves walk keys on their own. Keys split over workgroups
+// until there is one per CU, each wave keeping at least a 16-key tile.
+//   More rows: tiles of 64 rows (4 waves, up to 2 or more workgroups per CU)
+// or of 32 rows with the keys dealt to 4 wave groups (2 for f32 at D = 256, by
+// LDS; one workgroup per CU), and key splits where the rows leave CUs idle.
+// The least modelled time wins: rounds of workgroups x (16-key steps x time
+// per step + start and end), a merge 3 us plus its partials at 0.8 TB/s. Times
+// per step fitted to sweeps of both tilings and 1-8 splits over 16 shapes
+// (64-row tiles: alone on a CU / with company, which fills the waits; 32-row
+// tiles once per CU), e.g. 16 heads x 512 x 512 at D = 128: 50 us against
+// 29; 8 x 32 heads x 348 x 348 at D = 64: 73 against 135.
+static int attention_f32_launch(Runtime *rt, GqaTileArgs a, int64_t D, int64_t Dv, int kv_bf16,
+                                const AttnWorkspace *ext) {
+  const int64_t es = kv_bf16 ? 2 : 4, G = a.Hq / a.Hkv, R = G * a.Sq, NBH = (int64_t)a.NB * a.Hkv;
+  if (D != Dv || (D != 64 && D != 128 && D != 256) || a.Sk * D * es >= ((int64_t)1 << 31) ||
+      R >= ((int64_t)1 << 30) || ((uintptr_t)a.q | (uintptr_t)a.k | (uintptr_t)a.v | (uintptr_t)a.out) % 16 ||
+      (a.q_sb | a.q_sh | a.q_si | a.o_sb | a.o_sh | a.o_si | a.k_sb | a.k_sh | a.v_sb | a.v_sh) % 8 ||
+      env_int("RXW8_FORCE_GENERIC", 0))
+    return RXW8_UNIMPLEMENTED;
+  const int cus = rt->cus, forced = env_int("RXW8_ATTN_F32_SPLITS", 0);
+  const int64_t key_tiles = (a.Sk + 15) / 16;
+  int rg = 0;  // 0: the quad kernel; else 16-row groups of a tile workgroup
+  const int kg2 = D == 256 && !kv_bf16 ? 2 : 4;  // wave groups of the 32-row tiles
+  int64_t S = 1, units = NBH, rows = R;
+  if (R <= 8) {
+    S = std::max<int64_t>(1, std::min<int64_t>(cus / std::max<int64_t>(1, NBH), (key_tiles + 7) / 8));
+  } else {
+    const int di = D == 64 ? 0 : D == 128 ? 1 : 2;
+    static const double alone4[] = {1.1, 1.42, 2.8}, full4[] = {0.84, 1.2, 3.1}, ends4[] = {2, 3, 3};
+    static const double step2[] = {2.1, 2.8, 4.9}, ends2[] = {2.5, 4, 8};
+    const double tau2 = kv_bf16 ? (D == 64 ? 1.5 : step2[di]) : (D == 256 ? 3.1 : step2[di]);
+    const double keys = (double)a.Sk, mean = a.starts ? keys - 0.5 * (double)a.Sq : keys;  // longest, mean
+    double best = 0;
+    const int forced_rg = env_int("RXW8_ATTN_F32_RG", 0);
+    for (int g : {4, 2}) {
+      if ((forced_rg == 4 || forced_rg == 2) && g != forced_rg) continue;
+      const int64_t n = (R + 16 * g - 1) / (16 * g) * NBH, kg = g == 4 ? 1 : kg2;
+      for (int64_t s = 1; s <= 16 && (s == 1 || s * kg <= key_tiles); ++s) {
+        const double rounds = (double)((n * s + cus - 1) / cus), steps = 1.0 / (16.0 * (double)(s * kg));
+        const double one = g == 4 ? keys * steps * alone4[di] + ends4[di] : keys * steps * tau2 + ends2[di];
+        const double all = rounds * (g == 4 ? mean * steps * full4[di] + ends4[di] : mean * steps * tau2 + ends2[di]);
+        const double merge = s > 1 ? 3.0 + (double)(n * s * 16 * g * (4 + D) * 4) / 0.8e6 : 0.0;
+        const double t = std::max(one, all) + merge;
+        if (rg == 0 || t < best) best = t, rg = g, S = s;
+      }
+    }
+    a.tiles = (int)((R + 16 * rg - 1) / (16 * rg));
+    units = NBH * a.tiles;
+    rows = 16 * rg;
+  }
+  if (forced > 0) S = std::min<int64_t>(forced, 32);
+  S = std::min<int64_t>(S, 32);
+  const size_t per_split = (size_t)(units * rows) * (size_t)(4 + D) * sizeof(float);
+  // One workgroup per unit where the split workspace must not be used: in a
+  // stream capture (the graph would keep a pointer that a later, larger call
+  // frees), and for the decoder plan (slots), whose captured step runs the
+  // same plan as its eager one.
+  if (units > kF32UnitsMax || a.slots || (!ext && stream_capturing(rt))) S = 1;
+  if (S > 1) S = std::max<int64_t>(1, std::min<int64_t>(S, (int64_t)(kF32PartialMax / per_split)));
+  if (units * S >= ((int64_t)1 << 31)) return RXW8_UNIMPLEMENTED;
+  if (S > 1) {
+    const size_t need_p = per_split * (size_t)S, need_c = (size_t)units * sizeof(int);
+    if (ext) {
+      a.part = ext->partials;
+      a.counters = ext->counters;
+      if (need_p > ext->partial_bytes || need_c > ext->counter_bytes) S = 1;
+    } else if (ensure_workspace(rt, rt->scratch, need_p, false) ||
+               ensure_workspace(rt, rt->attn_counters, need_c, true)) {
+      S = 1;  // no memory for it: one workgroup per unit needs none
+    } else {
+      a.part = (float *)rt->scratch.ptr;
+      a.counters = (int *)rt->attn_counters.ptr;
+    }
+  }
+  a.nsplit = (int)S;
+  char kname[40];
+  const char *tn = kv_bf16 ? "bf16" : "f32";
+  if (rg == 0) {
+    const int ns = R <= 4 ? 1 : 2;
+    std::snprintf(kname, sizeof kname, "rxw8_gqa_quad_%s_d%d_s%d", tn, (int)D, ns);
+    return launch(rt, kname, dim3((unsigned)(units * S)), dim3(512), a, (size_t)32 * ns * (8 + 4 * D));
+  }
+  // LDS: each wave group's ring of 16-key K and V tiles (depth as in
+  // attention_f32.hip) and each wave's ring of mask values; the merges'
+  // records fit in it
+  const int kg = rg == 4 ? 1 : kg2, waves = rg * kg;
+  const int depth = rg == 4 ? (D == 256 && !kv_bf16 ? 2 : 3) : (D * es >= 512 ? 2 : 3);
+  std::snprintf(kname, sizeof kname, "rxw8_gqa_tile_%s_d%d_r%d", tn, (int)D, rg);
+  return launch(rt, kname, dim3((unsigned)(units * S)), dim3(64 * waves), a,
+                (size_t)kg * depth * 32 * D * es + (size_t)waves * depth * 1024);
+}
+
 int attention_launch(Runtime *rt, const void *q, int q_f32, const void *kc, const void *vc,
                      int cache_f32, const int32_t *lens, const int32_t *row_seq,
                      const float *mask, int64_t mask_sb, int64_t mask_sh, void *out, int out_f32,
@@ -1157,6 +1279,19 @@ int attention_launch(Runtime *rt, const void *q, int q_f32, const void *kc, cons
   }
   if (Lmax > 8192)
     return fail(RXW8_UNIMPLEMENTED, "decode attention: the generic kernel supports Lmax <= 8192");
+  {
+    GqaTileArgs t{};
+    t.q = q, t.k = kc, t.v = vc, t.mask = mask, t.out = out;
+    for (int i = 0; i < 4; ++i) t.bdim[i] = 1;
+    t.bdim[3] = R, t.mb[3] = mask_sb, t.msh = mask_sh, t.msj = 1;
+    t.q_sb = t.o_sb = Hq * D, t.q_sh = t.o_sh = D;
+    t.k_sb = t.v_sb = Hkv * Lmax * D, t.k_sh = t.v_sh = Lmax * D;
+    t.lens = lens, t.slots = row_seq;
+    t.NB = (int)R, t.Hq = (int)Hq, t.Hkv = (int)Hkv, t.Sq = 1, t.Sk = (int)Lmax;
+    t.scale = scale, t.q_bf16 = !q_f32, t.out_bf16 = !out_f32;
+    const int rc = attention_f32_launch(rt, t, D, D, !cache_f32, ext);
+    if (rc != RXW8_UNIMPLEMENTED) return rc;
+  }
   AttnGenericArgs a;
   a.q = q;
   a.kc = kc;
@@ -1187,6 +1322,26 @@ bool prefill_supported(int64_t Hq, int64_t Hkv, int64_t D, int cache_f32) {
   return !cache_f32 && D == 128 && Hkv > 0 && Hq % Hkv == 0 && (G == 1 || G == 2 || G == 4 || G == 8);
 }
 
+// The general GQA call: the f32 matrix-core kernels where they apply, else one
+// wave per output row.
+static int gqa_general_launch(Runtime *rt, const GqaGeneralArgs &a, int64_t NB) {
+  if (NB <= INT32_MAX) {
+    GqaTileArgs t{};
+    t.q = a.q, t.k = a.k, t.v = a.v, t.mask = a.mask, t.out = a.out;
+    for (int i = 0; i < 4; ++i) t.bdim[i] = a.bdim[i], t.mb[i] = a.mb[i];
+    t.msh = a.msh, t.msi = a.msi, t.msj = a.msj;
+    t.q_sb = a.q_sb, t.q_sh = a.q_sh, t.q_si = a.q_si;
+    t.o_sb = a.o_sb, t.o_sh = a.o_sh, t.o_si = a.o_si;
+    t.k_sb = a.k_sb, t.k_sh = a.k_sh, t.v_sb = a.v_sb, t.v_sh = a.v_sh;
+    t.starts = a.starts;
+    t.NB = (int)NB, t.Hq = a.Hq, t.Hkv = a.Hkv, t.Sq = a.Sq, t.Sk = a.Sk;
+    t.scale = a.scale, t.q_bf16 = a.q_bf16, t.out_bf16 = a.out_bf16;
+    const int rc = attention_f32_launch(rt, t, a.D, a.Dv, a.kv_bf16, nullptr);
+    if (rc != RXW8_UNIMPLEMENTED) return rc;
+  }
+  return launch(rt, "rxw8_gqa_general", dim3((unsigned)((a.rows + 3) / 4)), dim3(256), a);
+}
+
 // Causal prefill on the general GQA kernel: q / out element (b, i, h, d) at
 // b*sb + i*ss + h*sh + d, bf16 cache [B, Hkv, Lmax, D], row i of sequence b
 // seeing keys 0 .. clamp(starts[b], 0, Lmax - S) + i. Any head dim up to 512
@@ -1212,7 +1367,7 @@ static int prefill_general(Runtime *rt, const void *q, int q_bf16, int64_t q_sb,
   a.starts = starts;
   if ((a.rows + 3) / 4 >= ((int64_t)1 << 31))
     return fail(RXW8_UNIMPLEMENTED, "prefill attention: %lld rows exceed the grid", (long long)a.rows);
-  return launch(rt, "rxw8_gqa_general", dim3((unsigned)((a.rows + 3) / 4)), dim3(256), a);
+  return gqa_general_launch(rt, a, B);
 }
 
 int prefill_launch(Runtime *rt, const void *q, int q_f32, int64_t q_sb, int64_t q_ss, int64_t q_sh,
@@ -1742,7 +1897,7 @@ int rxw8_gqa_attention_into(rxw8_runtime *rt, rxw8_buffer *q, rxw8_buffer *k, rx
   if ((a.rows + 3) / 4 >= ((int64_t)1 << 31) || Sq > INT32_MAX || Sk > INT32_MAX)
     return fail(RXW8_UNIMPLEMENTED, "GQA: %lld rows exceed the kernel's grid", (long long)a.rows);
   std::lock_guard<std::recursive_mutex> g(rt->mu);
-  return launch(rt, "rxw8_gqa_general", dim3((unsigned)((a.rows + 3) / 4)), dim3(256), a);
+  return gqa_general_launch(rt, a, NB);
 }
 
 int rxw8_gqa_attention(rxw8_runtime *rt, rxw8_buffer *q, rxw8_buffer *k, rxw8_buffer *v,

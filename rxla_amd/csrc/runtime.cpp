@@ -18,6 +18,7 @@ extern const unsigned char rxw8_co_gemv[], rxw8_co_gemv_end[];
 extern const unsigned char rxw8_co_gemv_rc[], rxw8_co_gemv_rc_end[];
 extern const unsigned char rxw8_co_misc[], rxw8_co_misc_end[];
 extern const unsigned char rxw8_co_attention[], rxw8_co_attention_end[];
+extern const unsigned char rxw8_co_attention_f32[], rxw8_co_attention_f32_end[];
 extern const unsigned char rxw8_co_gemm[], rxw8_co_gemm_end[];
 extern const unsigned char rxw8_co_decoder[], rxw8_co_decoder_end[];
 extern const unsigned char rxw8_co_qwen35[], rxw8_co_qwen35_end[];
@@ -91,7 +92,7 @@ static int module_of(const char *kname) {
   } routes[] = {{"rxw8_gemv_rc_", 6}, {"rxw8_gemv_", 0},      {"rxw8_pack_tiles", 0},     {"rxw8_dequant", 1},
                 {"rxw8_linear_generic", 1}, {"rxw8_linear_f32_", 1}, {"rxw8_kv_update", 1},
                 {"rxw8_quantize_w8", 1},
-                {"rxw8_gqa_", 2},
+                {"rxw8_gqa_tile_", 7}, {"rxw8_gqa_quad_", 7}, {"rxw8_gqa_", 2},
                 {"rxw8_w8a16_gemm", 3}, {"rxw8_gemm_", 3},   {"rxw8_dec_", 4},
                 {"rxw8_q35_", 5}};
   for (const auto &r : routes)
@@ -151,17 +152,21 @@ void rt_free(Runtime *rt, void *ptr, size_t bytes) {
   rt->cached_bytes += bytes;
 }
 
-int ensure_workspace(Runtime *rt, Workspace &ws, size_t bytes, bool zero) {
-  if (ws.bytes >= bytes) return RXW8_OK;
-  // Growing synchronizes the stream and reallocates: not possible inside a
-  // stream capture (an XLA command buffer, a caller's graph). Such callers
-  // run the call once outside capture first, which sizes the workspace.
+bool stream_capturing(const Runtime *rt) {
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(rt->stream, &cs) != hipSuccess) {
     (void)hipGetLastError();
     cs = hipStreamCaptureStatusNone;
   }
-  if (cs != hipStreamCaptureStatusNone)
+  return cs != hipStreamCaptureStatusNone;
+}
+
+int ensure_workspace(Runtime *rt, Workspace &ws, size_t bytes, bool zero) {
+  if (ws.bytes >= bytes) return RXW8_OK;
+  // Growing synchronizes the stream and reallocates: not possible inside a
+  // stream capture (an XLA command buffer, a caller's graph). Such callers
+  // run the call once outside capture first, which sizes the workspace.
+  if (stream_capturing(rt))
     return fail(RXW8_FAILED_PRECONDITION,
                 "a workspace of %zu bytes (now %zu) must grow while the stream is being captured; "
                 "run the call once outside the capture first",
@@ -294,7 +299,8 @@ int rxw8_runtime_create(int device, rxw8_runtime **out) {
                {"gemm", rxw8_co_gemm, rxw8_co_gemm_end},
                {"decoder", rxw8_co_decoder, rxw8_co_decoder_end},
                {"qwen35", rxw8_co_qwen35, rxw8_co_qwen35_end},
-               {"gemv_rc", rxw8_co_gemv_rc, rxw8_co_gemv_rc_end}};
+               {"gemv_rc", rxw8_co_gemv_rc, rxw8_co_gemv_rc_end},
+               {"attention_f32", rxw8_co_attention_f32, rxw8_co_attention_f32_end}};
   for (auto &blob : blobs) {  // order = module indices of module_of()
     if (blob.end - blob.begin <= 0) {
       for (hipModule_t mm : rt->modules) (void)hipModuleUnload(mm);
