@@ -889,6 +889,85 @@ bool gemm_eligible(int64_t M, int64_t N, int64_t K, int64_t G) {
          N * K < (1LL << 32) && !env_int("RXW8_NO_GEMM", 0);
 }
 
+// Plan of the mid-size GEMM (kernels/gemm_mid.hip): rg (64 or 128 weight rows
+// per workgroup) and K splits by the least modelled time, in us: 3.5 fixed +
+// rounds x (512-k steps x time per step + 1.5), a split's reduce 2.5 plus its
+// partials at 4 TB/s. Times per step fitted to sweeps over 16 <= M <= 1024 and 1 to 16
+// splits (one workgroup per CU); f32 rows are converted in the kernel up to 64
+// of them, by a pass of their own beyond.
+struct MidPlan {
+  int rg = 0, ks = 1;
+  double us = 1e30;
+};
+// LDS of a workgroup: two buffers of 16 fj x 256 bf16 of x per wave group, and
+// the grouped scales of one split (the most groups that ceil(chunks / ks)
+// chunks can touch)
+static size_t mid_lds(int64_t fj, int rg, int ks, int64_t K, int64_t G) {
+  const int64_t span = (K / 256 + ks - 1) / ks * 256;
+  return (size_t)(4 * 16 * fj * 512) + (G == K ? 0 : (size_t)((span + G - 1) / G + 1) * 64 * rg * 4);
+}
+static bool mid_applies(const void *x, const void *w, const void *y, int64_t M, int64_t N, int64_t K, int64_t G) {
+  return N % 16 == 0 && K % 256 == 0 && K < ((int64_t)1 << 22) && (G == K || G % 64 == 0) &&
+         M * K * 2 < (1LL << 31) && N * K < (1LL << 32) && M <= (1 << 24) &&
+         ((uintptr_t)x | (uintptr_t)w | (uintptr_t)y) % 16 == 0 && env_int("RXW8_GEMM_MID", 1) &&
+         !env_int("RXW8_FORCE_GENERIC", 0);
+}
+static MidPlan plan_mid(const Runtime *rt, int64_t M, int64_t N, int64_t K, int64_t G, int x_f32, int y_mode) {
+  static const double step[2][4] = {{0.9, 1.4, 1.45, 1.85}, {1.6, 2.3, 2.7, 3.3}};
+  const int64_t fj = std::min<int64_t>(4, (M + 15) / 16), chunks = K / 256;
+  const int forced_rg = env_int("RXW8_MID_RG", 0), forced_ks = env_int("RXW8_MID_KS", 0);
+  MidPlan p;
+  for (int rg : {1, 2}) {
+    if (forced_rg && rg != forced_rg) continue;
+    const int64_t tiles = (M + 16 * fj - 1) / (16 * fj) * ((N + 64 * rg - 1) / (64 * rg));
+    double tau = step[rg - 1][fj - 1] * (G == K ? 1.0 : 1.1);
+    if (x_f32 && M <= 64) tau *= 1.25;
+    for (int ks : {1, 2, 3, 4, 6, 8, 12, 16}) {
+      if (ks > 1 && (2 * ks > chunks || y_mode == 2)) break;
+      if (forced_ks && ks != forced_ks && 2 * forced_ks <= chunks && y_mode != 2) continue;
+      if (mid_lds(fj, rg, ks, K, G) > rt->lds_max) continue;
+      const double wgs = (double)(tiles * ks) / rt->cus;
+      const double rounds = std::ceil(wgs);
+      const double iters = (double)((chunks + 2 * ks - 1) / (2 * ks));
+      double us = 3.5 + rounds * (iters * tau + 1.5) + (x_f32 ? (M <= 64 ? 0.5 : 3.0) : 0.0);
+      if (ks > 1) us += 2.5 + (ks + 1.0) * (double)M * N * 4.0 / 4e6;
+      if (us < p.us) p = MidPlan{rg, ks, us};
+    }
+  }
+  return p;
+}
+static int run_gemm_mid(Runtime *rt, MidPlan p, const void *x, int x_f32, const uint8_t *w, bool packed,
+                        const float *s, void *y, int y_f32, int64_t M, int64_t N, int64_t K, int64_t G,
+                        int y_mode) {
+  const int64_t fj = std::min<int64_t>(4, (M + 15) / 16);
+  const bool xf = x_f32 && M <= 64;
+  int rc;
+  // no room for the partials (a capture before the first eager call): one
+  // split needs none
+  if (p.ks > 1 && ensure_workspace(rt, rt->partials, (size_t)(p.ks * M * N) * 4, false)) {
+    if (mid_lds(fj, p.rg, 1, K, G) > rt->lds_max) return RXW8_UNIMPLEMENTED;
+    p.ks = 1;
+  }
+  if (x_f32 && !xf) {
+    if ((rc = ensure_workspace(rt, rt->xcast, (size_t)(M * K) * 2, false))) return rc;
+    CastArgs c{(const float *)x, (uint16_t *)rt->xcast.ptr, M * K};
+    if ((rc = launch(rt, "rxw8_gemm_cast_x", dim3(grid_for(M * K / 4 + 1, 256, 4096)), dim3(256), c)))
+      return rc;
+    x = rt->xcast.ptr;
+  }
+  const int64_t tiles = (M + 16 * fj - 1) / (16 * fj) * ((N + 64 * p.rg - 1) / (64 * p.rg));
+  GemmArgs a{(const uint16_t *)x, w, s, y, (int)M, (int)N, (int)K, (int)G, y_f32, y_mode, packed ? 1 : 0, 0, p.ks,
+             p.ks > 1 ? (float *)rt->partials.ptr : nullptr};
+  char kname[40];
+  std::snprintf(kname, sizeof kname, "rxw8_gemm_mid_m%d_r%d%s%s", (int)fj, p.rg, G == K ? "" : "_g", xf ? "_xf" : "");
+  if ((rc = launch(rt, kname, dim3((unsigned)((tiles * p.ks + 7) / 8 * 8)), dim3(512), a,
+                   mid_lds(fj, p.rg, p.ks, K, G))))
+    return rc;
+  if (p.ks == 1) return RXW8_OK;
+  SplitkReduceArgs r{(const float *)rt->partials.ptr, nullptr, y, (int)M, (int)N, p.ks, y_f32, y_mode};
+  return launch(rt, "rxw8_gemv_splitk_reduce", dim3(grid_for(M * N / 4, 256, 4096)), dim3(256), r);
+}
+
 // Requires gemm_eligible(): one scale per weight row and 64-deep k tile.
 static int run_gemm(Runtime *rt, const void *x, int x_f32, const uint8_t *w, bool packed,
                     const float *s, void *y, int y_f32, int64_t M, int64_t N, int64_t K,
@@ -955,6 +1034,17 @@ static int run_gemm(Runtime *rt, const void *x, int x_f32, const uint8_t *w, boo
     }
   }
   if (!best) return fail(RXW8_INVALID_ARGUMENT, "no GEMM tiling for N=%lld", (long long)N);
+  // Few rows or few tiles: the mid-size GEMM where its modelled time is the
+  // smaller (these tilings' calls measure 5 to 8 us above their model at small
+  // sizes: 655 x 2048 x 2048 31 us against 18, 240 x 1024 x 6144 38 against
+  // 19; 338 x 6144 x 4096 47 against 54, 512 x 12288 x 4096 71 against 86).
+  if (!forced && !forced_ks && env_int("RXW8_GEMM_BF16W", -1) != 1 && mid_applies(x, w, y, M, N, K, G)) {
+    const MidPlan p = plan_mid(rt, M, N, K, G, 0, y_mode);
+    if (p.rg && (p.us < best_t * 1e6 + 3.0 || env_int("RXW8_GEMM_MID", 1) > 1)) {
+      rc = run_gemm_mid(rt, p, x, 0, w, packed, s, y, y_f32, M, N, K, G, y_mode);
+      if (rc != RXW8_UNIMPLEMENTED) return rc;
+    }
+  }
   const int64_t tiles = (M + best->tm - 1) / best->tm * (N / best->tn);
   const int64_t per_xcd = (tiles + 7) / 8;
   // Long inputs: dequantise the weights once into a bf16 workspace (a
@@ -1000,6 +1090,24 @@ int qlinear_launch(Runtime *rt, const void *x, int x_f32, const uint8_t *w, bool
                    int64_t G, int compute_bf16, int y_mode) {
   if (M == 0) return RXW8_OK;
   if (y_mode == 1) y_f32 = 1;  // the residual y is f32 (row offsets of M chunks use it)
+  // Between the GEMV (one weight stream per 16 or 32 rows) and the 128- and
+  // 256-row GEMM tiles (run_gemm makes that choice): the mid-size GEMM where its
+  // modelled time is below the GEMV's, in us per chunk of rows fitted to the
+  // same sweep: 4 + 0.42 per MB of weights per 32 bf16 rows (5 + 0.45 for
+  // f32), 7 + 0.24 for up to 16 f32 rows (bf16 rows of that count are staged
+  // by LDS DMA and stay). 48 x 6144 x 4096: 29 us against 14; 8 x 12288 x
+  // 2048 f32: 12.6 against 9.1; 32 x 2048 x 2048: 6.4 against 7.4.
+  if (compute_bf16 && y_mode != 2 && M > (x_f32 ? 4 : 16) && !gemm_eligible(M, N, K, G) &&
+      mid_applies(x, w, y, M, N, K, G)) {
+    const double mb = (double)(N * K) * 1e-6;
+    const double gemv = M <= 16 ? 7.0 + 0.24 * mb
+                                : (double)((M + 31) / 32) * (x_f32 ? 5.0 + 0.45 * mb : 4.0 + 0.42 * mb);
+    const MidPlan p = plan_mid(rt, M, N, K, G, x_f32, y_mode);
+    if (p.rg && (p.us < gemv || env_int("RXW8_GEMM_MID", 1) > 1)) {
+      const int rc = run_gemm_mid(rt, p, x, x_f32, w, packed, s, y, y_f32, M, N, K, G, y_mode);
+      if (rc != RXW8_UNIMPLEMENTED) return rc;
+    }
+  }
   if (packed) {
     if (compute_bf16 && gemm_eligible(M, N, K, G))
       return run_gemm(rt, x, x_f32, w, true, s, y, y_f32, M, N, K, G, y_mode);

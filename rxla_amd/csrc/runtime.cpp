@@ -20,6 +20,7 @@ extern const unsigned char rxw8_co_misc[], rxw8_co_misc_end[];
 extern const unsigned char rxw8_co_attention[], rxw8_co_attention_end[];
 extern const unsigned char rxw8_co_attention_f32[], rxw8_co_attention_f32_end[];
 extern const unsigned char rxw8_co_gemm[], rxw8_co_gemm_end[];
+extern const unsigned char rxw8_co_gemm_mid[], rxw8_co_gemm_mid_end[];
 extern const unsigned char rxw8_co_decoder[], rxw8_co_decoder_end[];
 extern const unsigned char rxw8_co_qwen35[], rxw8_co_qwen35_end[];
 }
@@ -93,7 +94,7 @@ static int module_of(const char *kname) {
                 {"rxw8_linear_generic", 1}, {"rxw8_linear_f32_", 1}, {"rxw8_kv_update", 1},
                 {"rxw8_quantize_w8", 1},
                 {"rxw8_gqa_tile_", 7}, {"rxw8_gqa_quad_", 7}, {"rxw8_gqa_", 2},
-                {"rxw8_w8a16_gemm", 3}, {"rxw8_gemm_", 3},   {"rxw8_dec_", 4},
+                {"rxw8_w8a16_gemm", 3}, {"rxw8_gemm_mid_", 8}, {"rxw8_gemm_", 3},   {"rxw8_dec_", 4},
                 {"rxw8_q35_", 5}};
   for (const auto &r : routes)
     if (std::strncmp(kname, r.prefix, std::strlen(r.prefix)) == 0) return r.module;
@@ -300,7 +301,8 @@ int rxw8_runtime_create(int device, rxw8_runtime **out) {
                {"decoder", rxw8_co_decoder, rxw8_co_decoder_end},
                {"qwen35", rxw8_co_qwen35, rxw8_co_qwen35_end},
                {"gemv_rc", rxw8_co_gemv_rc, rxw8_co_gemv_rc_end},
-               {"attention_f32", rxw8_co_attention_f32, rxw8_co_attention_f32_end}};
+               {"attention_f32", rxw8_co_attention_f32, rxw8_co_attention_f32_end},
+               {"gemm_mid", rxw8_co_gemm_mid, rxw8_co_gemm_mid_end}};
   for (auto &blob : blobs) {  // order = module indices of module_of()
     if (blob.end - blob.begin <= 0) {
       for (hipModule_t mm : rt->modules) (void)hipModuleUnload(mm);

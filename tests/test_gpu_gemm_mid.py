@@ -1,0 +1,80 @@
+"""The mid-size W8A16 GEMM (a few dozen to a few hundred rows) at the edges of
+its tiles, against the CPU oracle on every plan: 16-row fragments, 64-row
+tiles, 64- and 128-channel tiles, K splits (also uneven ones and more wave
+groups than chunks), grouped scales that straddle the 256-wide chunks, f32 and
+bf16 rows, both weight layouts. Tolerance: the operands are the oracle's bf16
+values and the sums f32, so results agree to one bf16 rounding (2^-8 of the
+element) with most bits equal; normwise 1e-2 / 2."""
+import numpy as np
+import pytest
+
+import oracle
+from conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def rx():
+    import rxla_amd
+    return rxla_amd
+
+
+def run(rt, x, u8, s, xd, packed, yd):
+    r = rx()
+    xb = rt.buffer(oracle.bf16_bits(x), r.DType.BF16) if xd == "bf16" else rt.buffer(x)
+    wb = rt.buffer(u8)
+    if packed:
+        wb = r.pack_weight(rt, wb)
+    y = r.quantized_linear(rt, xb, wb, rt.buffer(s), r.DType.BF16,
+                           r.DType.F32 if yd == "f32" else r.DType.BF16).to_numpy()
+    return r.bf16_to_f32(y) if yd == "bf16" else y
+
+
+@pytest.mark.parametrize("m,n,k,g", [(17, 64, 256, 256), (32, 48, 512, 64), (48, 208, 1024, 128),
+                                     (64, 128, 768, 192), (65, 256, 512, 512), (100, 80, 1280, 320),
+                                     (130, 384, 2304, 128), (5, 144, 512, 512)])
+@pytest.mark.parametrize("rg,ks", [(1, 1), (2, 1), (1, 2), (2, 3)])
+def test_tiles_against_the_oracle(rt, monkeypatch, m, n, k, g, rg, ks):
+    monkeypatch.setenv("RXW8_GEMM_MID", "2")
+    monkeypatch.setenv("RXW8_MID_RG", str(rg))
+    monkeypatch.setenv("RXW8_MID_KS", str(ks))
+    rng = np.random.default_rng(m + n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    u8, s = oracle.quantize_w8((rng.standard_normal((n, k)) * 0.02).astype(np.float32), g)
+    want = oracle.quantized_linear(x, u8, s, oracle.COMPUTE_BF16)
+    for xd in ("f32", "bf16") if m > 16 else ("f32",):
+        for packed in (False, True) if m <= 64 or n % 128 == 0 else (False,):
+            for yd in ("f32", "bf16"):
+                got = run(rt, x, u8, s, xd, packed, yd)
+                assert rel_err(got, want) <= 5e-3
+                # one bf16 step, at most, per element
+                assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 0.05)) <= 2.0 ** -7
+
+
+@pytest.mark.parametrize("m,n,k", [(48, 6144, 4096), (33, 4096, 1024), (100, 2048, 6144), (200, 1040, 512)])
+def test_default_plans(rt, monkeypatch, m, n, k):
+    """The default rule's choice against the paths it replaces (one bf16 step)."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    u8, s = oracle.quantize_w8((rng.standard_normal((n, k)) * 0.02).astype(np.float32), 128)
+    got = run(rt, x, u8, s, "f32", False, "f32")
+    again = run(rt, x, u8, s, "f32", False, "f32")
+    np.testing.assert_array_equal(got, again)
+    monkeypatch.setenv("RXW8_GEMM_MID", "0")
+    want = run(rt, x, u8, s, "f32", False, "f32")
+    rms = np.sqrt(np.mean(want * want))
+    assert np.max(np.abs(got - want) / np.maximum(np.abs(want), rms)) <= 2.0 ** -7
+    assert np.mean(got != want) < 0.05
+
+
+def test_rows_and_scales_that_are_not_numbers_stay_in_their_row(rt):
+    """NaN and infinite activations reach their own row's outputs alone."""
+    rng = np.random.default_rng(2)
+    x = rng.standard_normal((40, 2048)).astype(np.float32)
+    u8, s = oracle.quantize_w8((rng.standard_normal((4096, 2048)) * 0.02).astype(np.float32), 2048)
+    clean = run(rt, x, u8, s, "bf16", False, "f32")
+    x[7, 100], x[39, 2047] = np.nan, np.inf
+    got = run(rt, x, u8, s, "bf16", False, "f32")
+    keep = np.array([i for i in range(40) if i not in (7, 39)])
+    np.testing.assert_array_equal(got[keep], clean[keep])
+    assert np.isnan(got[7]).all() and not np.isfinite(got[39]).any()
