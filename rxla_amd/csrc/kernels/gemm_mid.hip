@@ -286,6 +286,165 @@ __device__ __forceinline__ void gemm_mid(const GemmArgs &a) {
     }
 }
 
+// ---- F32 compute (gemm.hip rxw8_gemm_f32c's product and contract) -------------
+//   y[m, n] = sum_g s[n, g] * sum_{k in g} (xh[m, k] + xl[m, k]) * (u8[n, k] - 128)
+// on the same scheme: weights global -> registers -> exact bf16 codes, each
+// wave its own 64 weight rows; 64 (16 FJ) rows of xh and xl through LDS in
+// chunks of 128 k. 256 x 64 output tiles of 4 waves, two workgroups per CU
+// with waits and barriers of their own, where the 256 x 128 tiles of gemm.hip
+// hold a CU each with 8 waves in lockstep and, at a few hundred rows, leave
+// half the CUs without a tile or split K into a reduce pass. A scale group's
+// f32 sum is scaled into the total at the group's end (a split's part of a
+// group scales its own part).
+struct LinearF32GemmArgs {
+  const uint16_t *xh, *xl;  // [M, K] bf16 hi / lo parts of x
+  const uint8_t *w;         // [N, K] u8 codes, or packed [N/16, K/64, 1024]
+  const float *scale;       // [N, K / G]
+  float *y;                 // [M, N]
+  int M, N, K, G;
+  int y_mode;               // 0: y = result; 1: y += result
+  int w_packed;
+  int ksplit;               // 1, or the number of K splits
+  float *ws;                // [ksplit, M, N] f32 partials when ksplit > 1
+};
+
+// Four codes u -> the bf16 pairs of u - 128 (exact): the top bit flipped they
+// are signed bytes, one sign-extending conversion each
+__device__ __forceinline__ uint2 signed_bf16x4(uint32_t w) {
+  w ^= 0x80808080u;
+  const float f0 = (float)(int8_t)w, f1 = (float)(int8_t)(w >> 8);
+  const float f2 = (float)(int8_t)(w >> 16), f3 = (float)((int32_t)w >> 24);
+  return uint2{pack_bf16x2(f0, f1), pack_bf16x2(f2, f3)};
+}
+
+template <int FJ>
+__device__ __forceinline__ void gemm_f32m(const LinearF32GemmArgs &a) {
+  constexpr int RG = 4, TM = 16 * FJ, TN = 256, CKF = 128, RB = CKF * 2, XB = TM * RB;
+  constexpr int XDMA = XB / 1024 / 4;  // LDS-DMA instructions per wave, part and chunk
+  extern __shared__ __attribute__((aligned(1024))) char smem[];  // [2 buffers][xh | xl], scales
+  const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  const int wn = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tiles_m = (a.M + TM - 1) / TM, tiles_n = (a.N + TN - 1) / TN, ntiles = tiles_m * tiles_n;
+  const int per_xcd = (ntiles * a.ksplit + 7) / 8;
+  const int t_all = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
+  if (t_all >= ntiles * a.ksplit) return;
+  const int split = t_all / ntiles, t = t_all - split * ntiles;
+  constexpr int GN = 8;  // n tiles per tile-order group (n fastest): an XCD's 64 tiles are about 8 x 8
+  const int group = t / (GN * tiles_m), in = t - group * GN * tiles_m, gw = min(GN, tiles_n - group * GN);
+  const int nt = (group * GN + in % gw) * TN, n0 = nt + wn * 64, m0 = in / gw * TM;
+  const int KT = a.K / 64, chunks = a.K / CKF, ng = a.K / a.G;
+  const int cb = split * chunks / a.ksplit, ce = (split + 1) * chunks / a.ksplit, last = ce - 1;
+  const uint32_t gk = (uint32_t)a.G / 64, ginv = gk > 1 ? 0xffffffffu / gk + 1 : 0;
+  auto group_of = [&](int step) { return (int)(gk > 1 ? __umulhi((uint32_t)step, ginv) : (uint32_t)step); };
+  float *scl = (float *)(smem + 4 * XB);  // [group][row], the split's groups
+  const int g_lo = group_of(2 * cb), g_n = group_of(2 * ce - 1) + 1 - g_lo;
+
+  uint32_t xoff[XDMA];
+#pragma unroll
+  for (int i = 0; i < XDMA; ++i) {
+    const int row = 4 * (wn * XDMA + i) + (lane >> 4);
+    const int m = min(m0 + row, a.M - 1);  // rows past M repeat the last row (not stored)
+    xoff[i] = (uint32_t)m * (uint32_t)a.K * 2u + ((uint32_t)((lane & 15) ^ (row & 15)) << 4);
+  }
+  auto issue_x = [&](int c, int buf) {
+#pragma unroll
+    for (int i = 0; i < XDMA; ++i) {
+      const uint32_t l = lds_addr(smem + buf * 2 * XB + (wn * XDMA + i) * 1024);
+      dma16(a.xh, xoff[i] + (uint32_t)c * RB, l);
+      dma16(a.xl, xoff[i] + (uint32_t)c * RB, l + XB);
+    }
+  };
+  const int kstride = a.w_packed ? 1024 : 64;
+  uint32_t woff[RG];
+#pragma unroll
+  for (int g = 0; g < RG; ++g) {
+    const int n = min(n0 + 16 * g + r16, a.N - 1);
+    woff[g] = a.w_packed ? (uint32_t)(n >> 4) * (uint32_t)KT * 1024u + (uint32_t)((n & 15) + 16 * kq) * 16u
+                         : (uint32_t)n * (uint32_t)a.K + (uint32_t)kq * 16u;
+  }
+  u32x4 w[2][RG];
+  auto load_w = [&](int c, int s) {
+#pragma unroll
+    for (int g = 0; g < RG; ++g)
+      w[s][g] = *(const u32x4 *)(a.w + woff[g] + (uint32_t)(2 * c + s) * (uint32_t)kstride);
+  };
+  issue_x(cb, 0);
+  load_w(cb, 0);
+  load_w(cb, 1);
+  for (int e = threadIdx.x; e < TN * g_n; e += 256) {
+    const int row = e / g_n, g = e - row * g_n;
+    scl[g * TN + row] = a.scale[(int64_t)min(nt + row, a.N - 1) * ng + g_lo + g];
+  }
+  f32x4 acc[RG][FJ], tot[RG][FJ];
+#pragma unroll
+  for (int g = 0; g < RG; ++g)
+#pragma unroll
+    for (int j = 0; j < FJ; ++j) acc[g][j] = tot[g][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int c = cb; c < ce; ++c) {
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // chunk c is here; the other buffer is free
+    const char *xb = smem + ((c - cb) & 1) * 2 * XB;
+    const int cn = min(c + 1, last);
+    issue_x(cn, (c + 1 - cb) & 1);
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      u32x4 wf[RG][2];
+#pragma unroll
+      for (int g = 0; g < RG; ++g)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const uint2 lo = signed_bf16x4(w[s][g][2 * h]), hi = signed_bf16x4(w[s][g][2 * h + 1]);
+          wf[g][h] = u32x4{lo.x, lo.y, hi.x, hi.y};
+        }
+      load_w(cn, s);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        bf16x8 xf[2][FJ];
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int j = 0; j < FJ; ++j)
+            xf[p][j] = as_bf16x8(*(const u32x4 *)(xb + p * XB + (16 * j + r16) * RB + (((8 * s + 2 * kq + h) ^ r16) << 4)));
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+          for (int g = 0; g < RG; ++g)
+#pragma unroll
+            for (int j = 0; j < FJ; ++j) acc[g][j] = mfma16x16x32(as_bf16x8(wf[g][h]), xf[p][j], acc[g][j]);
+      }
+      const int step = 2 * c + s, gi = group_of(step);
+      if (step + 1 == 2 * ce || group_of(step + 1) != gi) {  // (uniform) the group's, or the split's, end
+#pragma unroll
+        for (int g = 0; g < RG; ++g) {
+          const f32x4 sv = *(const f32x4 *)(scl + (gi - g_lo) * TN + wn * 64 + 16 * g + 4 * kq);
+#pragma unroll
+          for (int j = 0; j < FJ; ++j) {
+            tot[g][j] += sv * acc[g][j];
+            acc[g][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
+        }
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies past the last chunk
+  // lane holds D[n = 16 g + 4 kq + e][m = 16 j + r16]
+#pragma unroll
+  for (int j = 0; j < FJ; ++j) {
+    const int m = m0 + 16 * j + r16;
+    if (m >= a.M) continue;
+#pragma unroll
+    for (int g = 0; g < RG; ++g) {
+      const int n = n0 + 16 * g + 4 * kq;
+      if (n >= a.N) continue;
+      if (a.ksplit > 1) {
+        *(f32x4 *)(a.ws + ((int64_t)split * a.M + m) * a.N + n) = tot[g][j];
+      } else {
+        f32x4 *yp = (f32x4 *)(a.y + (int64_t)m * a.N + n);
+        *yp = a.y_mode == 1 ? *yp + tot[g][j] : tot[g][j];
+      }
+    }
+  }
+}
+
 }  // namespace
 
 // Launch contract (checked by the host): x bf16, or f32 for the _xf kernels
@@ -312,3 +471,14 @@ RXW8_GEMM_MID_FJ(1)
 RXW8_GEMM_MID_FJ(2)
 RXW8_GEMM_MID_FJ(3)
 RXW8_GEMM_MID_FJ(4)
+
+// Launch contract as rxw8_gemm_f32c (gemm.hip), and: K % 128 == 0, ksplit <= K
+// / 128, LDS 4 * 16 FJ * 256 bytes + the split's groups x 256 floats; 256
+// threads; grid = 8 * ceil(tiles * ksplit / 8).
+#define RXW8_GEMM_F32M(FJ)                                                                      \
+  extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))    \
+      rxw8_gemm_mid_f32_m##FJ(LinearF32GemmArgs a) {                                           \
+    gemm_f32m<FJ>(a);                                                                          \
+  }
+RXW8_GEMM_F32M(2)
+RXW8_GEMM_F32M(4)

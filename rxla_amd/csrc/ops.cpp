@@ -719,12 +719,67 @@ int f32_gemm_operands(Runtime *rt, int64_t M, int64_t K, uint16_t **hi, uint16_t
   return RXW8_OK;
 }
 
+// F32-compute tiles of 256 x 64 (or 32) with the weights in registers, two
+// workgroups per CU (kernels/gemm_mid.hip): tile rows / 16, and K splits by
+// the least modelled time (us per 128-k chunk of a workgroup alone on its CU
+// and of two sharing it, a split's reduce 2.5 plus its partials at 2.5 TB/s;
+// fitted to sweeps of 1 to 12 splits). ks 0 where they do not apply (K % 128);
+// elsewhere they beat or tie the 256 x 128 tiles of gemm.hip from 17 to 2048
+// rows: 500 x 7168 x 1024 47.8 -> 30.8 us, 330 x 8320 x 1024 45.2 -> 30.3, 17 x
+// 1024 x 3584 21.8 -> 14.5, 500 x 248320 x 1024 618 -> 603.
+struct F32MidPlan {
+  int fj = 4, ks = 0;
+};
+static size_t f32_mid_lds(int64_t fj, int ks, int64_t K, int64_t G) {
+  const int64_t span = (K / 128 + ks - 1) / ks * 128;
+  return (size_t)(4 * 16 * fj * 256) + (size_t)((span + G - 1) / G + 1) * 256 * 4;
+}
+static F32MidPlan plan_f32_mid(const Runtime *rt, int64_t M, int64_t N, int64_t K, int64_t G) {
+  F32MidPlan p;
+  const int env = env_int("RXW8_F32_MID", 1), forced = env_int("RXW8_F32_MID_KS", 0);
+  if (!env || K % 128 || K >= ((int64_t)1 << 22) || env_int("RXW8_F32_GEMM_KSPLIT", 0)) return p;
+  p.fj = M <= 32 ? 2 : 4;
+  const int64_t tiles = (M + 16 * p.fj - 1) / (16 * p.fj) * ((N + 255) / 256), chunks = K / 128;
+  double best = 0;
+  for (int ks : {1, 2, 3, 4, 6, 8, 12}) {
+    if (ks > chunks || f32_mid_lds(p.fj, ks, K, G) * 2 > rt->lds_max) continue;
+    if (forced && forced != ks) continue;
+    // one or two workgroups per CU: time of a 128-k chunk alone and in a pair
+    const int64_t wgs = tiles * ks, per = (chunks + ks - 1) / ks;
+    const double alone = p.fj == 2 ? 1.5 : 2.4, pair = p.fj == 2 ? 2.3 : 3.7;
+    double us = wgs <= rt->cus ? (double)per * alone
+                               : (double)((wgs + 2 * rt->cus - 1) / (2 * rt->cus)) * (double)per * pair;
+    if (ks > 1) us += 2.5 + (ks + 1.0) * (double)M * N * 4.0 / 2.5e6;
+    if (p.ks == 0 || us < best) best = us, p.ks = ks;
+  }
+  return p;
+}
+
 // (x == nullptr: the caller has written x's parts into f32_gemm_operands'
 // buffers, e.g. the Qwen3.5 RMSNorm; no split launch)
 static int run_linear_f32_gemm(Runtime *rt, const float *x, const uint8_t *w, bool packed,
                                const float *scale, float *y, int64_t M, int64_t N, int64_t K,
                                int64_t G, int y_mode) {
   if (!f32_gemm_applies(w, y, M, N, K, G)) return RXW8_UNIMPLEMENTED;
+  const F32MidPlan mp = plan_f32_mid(rt, M, N, K, G);
+  if (mp.ks > 0) {
+    uint16_t *xh, *xl;
+    int rc = f32_gemm_operands(rt, M, K, &xh, &xl);
+    if (rc) return rc;
+    if (mp.ks > 1 && (rc = ensure_workspace(rt, rt->partials, (size_t)(mp.ks * M * N) * 4, false))) return rc;
+    SplitXArgs sx{x, xh, xl, M * K};
+    if (x && (rc = launch(rt, "rxw8_gemm_split_x", dim3(grid_for(M * K / 4, 256, 4096)), dim3(256), sx)))
+      return rc;
+    LinearF32GemmArgs a{xh, xl, w, scale, y, (int)M, (int)N, (int)K, (int)G, y_mode, packed ? 1 : 0,
+                        mp.ks, mp.ks > 1 ? (float *)rt->partials.ptr : nullptr};
+    const int64_t mt = (M + 16 * mp.fj - 1) / (16 * mp.fj) * ((N + 255) / 256) * mp.ks;
+    if ((rc = launch(rt, mp.fj == 2 ? "rxw8_gemm_mid_f32_m2" : "rxw8_gemm_mid_f32_m4",
+                     dim3((unsigned)((mt + 7) / 8 * 8)), dim3(256), a, f32_mid_lds(mp.fj, mp.ks, K, G))))
+      return rc;
+    if (mp.ks == 1) return RXW8_OK;
+    F32ReduceArgs r{(const float *)rt->partials.ptr, y, M * N, mp.ks, y_mode};
+    return launch(rt, "rxw8_gemm_f32c_reduce", dim3(grid_for(M * N / 4, 256, 4096)), dim3(256), r);
+  }
   const int64_t tiles = (M + 127) / 128 * ((N + 255) / 256);
   // split units: scale groups, or the k tiles of a single group
   const int64_t ng = K / G, units = ng > 1 ? ng : K / 64, upt = ng > 1 ? G / 64 : 1;

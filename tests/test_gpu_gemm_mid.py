@@ -78,3 +78,34 @@ def test_rows_and_scales_that_are_not_numbers_stay_in_their_row(rt):
     keep = np.array([i for i in range(40) if i not in (7, 39)])
     np.testing.assert_array_equal(got[keep], clean[keep])
     assert np.isnan(got[7]).all() and not np.isfinite(got[39]).any()
+
+
+@pytest.mark.parametrize("m,n,k,g", [(17, 256, 128, 64), (33, 272, 384, 128), (64, 512, 768, 192),
+                                     (65, 48, 640, 640), (130, 304, 1024, 128), (200, 256, 1280, 64)])
+@pytest.mark.parametrize("ks", [1, 2, 3])
+@pytest.mark.parametrize("packed", [False, True])
+def test_f32_compute_tiles(rt, monkeypatch, m, n, k, g, ks, packed):
+    """The F32-compute tiles of the same file, 32- and 64-row tiles, splits
+    that cut scale groups, against the oracle's float64 result: x enters as
+    bf16 hi + lo parts (2^-17 of the value), the sums are f32."""
+    monkeypatch.setenv("RXW8_F32_MID_KS", str(min(ks, k // 128)))
+    r = rx()
+    rng = np.random.default_rng(m + k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    u8, s = oracle.quantize_w8((rng.standard_normal((n, k)) * 0.02).astype(np.float32), g)
+    wb = rt.buffer(u8)
+    if packed:
+        wb = r.pack_weight(rt, wb)
+    got = r.quantized_linear(rt, rt.buffer(x), wb, rt.buffer(s), r.DType.F32, r.DType.F32).to_numpy()
+    want = x.astype(np.float64) @ (((u8.astype(np.float64) - 128).reshape(n, k // g, g)
+                                    * s.astype(np.float64)[:, :, None]).reshape(n, k)).T
+    assert rel_err(got, want) <= 1e-5
+    # whole-number inputs that need the lo part: exact
+    xi = rng.integers(-2000, 2001, (m, k)).astype(np.float32)
+    si = np.ones_like(s)
+    ui = rng.integers(126, 131, (n, k)).astype(np.uint8)
+    wi = rt.buffer(ui)
+    if packed:
+        wi = r.pack_weight(rt, wi)
+    yi = r.quantized_linear(rt, rt.buffer(xi), wi, rt.buffer(si), r.DType.F32, r.DType.F32).to_numpy()
+    np.testing.assert_array_equal(yi, xi.astype(np.float64) @ (ui.astype(np.float64) - 128).T)
