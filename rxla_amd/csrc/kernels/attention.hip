@@ -1155,15 +1155,30 @@ __device__ __forceinline__ uint32_t lds_u32(const uint16_t *p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t *)p;
 }
 
-// R row tiles per wave: as attn_prefill_wh, but wave w owns rows
-// 16 R (w % 4) .. + 16 R - 1 of a workgroup's 64 R query rows, as R 16-row
-// tiles of one head. Every K and V^T fragment read from LDS then feeds R
-// tiles' MFMAs (the LDS reads per block per wave stay 32 KiB, the matrix work
-// grows R-fold), and each staged K/V block serves 64 R rows. Same arithmetic
-// per (row, head) as attn_prefill.
-template <int G, int R>
+// (constant arguments of the generic lambdas below)
+struct Yes { static constexpr bool value = true; };
+struct No { static constexpr bool value = false; };
+
+// R row tiles per wave: wave w owns rows 16 R (w % 4) .. + 16 R - 1 of a
+// workgroup's 64 R query rows, as R 16-row tiles of one head. Every K and V^T
+// fragment read from LDS feeds R tiles' MFMAs, and each staged K/V block
+// serves 64 R rows.
+//
+// A block is two halves: matrix (PV of the block before, QK of this one) and
+// vector (the softmax). A SIMD holds one wave of each head, and the second
+// head's waves run half a step behind the first's, so one wave's softmax runs
+// under the other's MFMAs; a barrier per half keeps them there. All waves in
+// step (one barrier a block) measured 65.4 us against 61.0 at 2048 rows,
+// batch 1, 32 heads. LDS reads a few fragments ahead of their MFMAs, the
+// copies in rings of 4 blocks, a bf16 q without a lo part (the scale goes to
+// the scores instead: two thirds of the matrix work), no row maximum unless
+// the reference moves, waves past the last row idle: 4 x 777 rows at 500 on,
+// 32 heads, 91 -> 62 us; 4 x 2048 rows 220 -> 170. What bounds it now: the
+// LDS reads of a matrix half (32 KiB a wave; ~1900 cycles a half against 1024
+// of MFMA).
+template <int G, int R, bool LO>
 __device__ void attn_prefill_rt(const PrefillArgs &a) {
-  extern __shared__ __attribute__((aligned(16))) uint16_t pf_lds[];  // [2][K block] [2][V block]
+  extern __shared__ __attribute__((aligned(16))) uint16_t pf_lds[];  // [NB][K block] [NB][V block]
   constexpr int QROWS = 64 * R;   // query rows per workgroup
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, g4 = lane >> 4;
@@ -1174,7 +1189,9 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
   const int per_qb = a.B * a.Hkv * HP;
   const int qb = a.nqb - 1 - (int)(blockIdx.x / per_qb);
   const int rem3 = blockIdx.x - (a.nqb - 1 - qb) * per_qb;
-  const int hp = HP > 1 ? rem3 % HP : 0, rem = HP > 1 ? rem3 / HP : rem3;
+  // (a kv head's workgroups a multiple of B Hkv apart: on one XCD's L2 where
+  // that is a multiple of 8)
+  const int hp = rem3 / (a.B * a.Hkv), rem = rem3 - hp * (a.B * a.Hkv);
   const int b = rem / a.Hkv, kvh = rem - (rem / a.Hkv) * a.Hkv;
   int start = a.starts[b];  // clamped so rows sit in [0, Lmax) (host: S <= Lmax)
   start = start < 0 ? 0 : (start > a.Lmax - a.S ? a.Lmax - a.S : start);
@@ -1188,38 +1205,86 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
   for (int r = 0; r < R; ++r) my_pos[r] = start + min(i0 + 16 * r + col, a.S - 1);
   const int wave_last = start + min(i0 + 16 * R - 1, a.S - 1);
   const int hq = kvh * G + hp * HW + head;
-  const float c_exp = a.scale * 1.4426950408889634f;  // scale * log2(e)
+  // Block staging by LDS DMA (no registers held across the block), both
+  // operands in rings of NB blocks and row-major with 16-byte chunks
+  // XOR-swizzled by row (the lane writing LDS chunk slot c' of row r fetches
+  // global chunk c' ^ f(r)): K with f(r) = r & 15 (conflict-free fragment
+  // reads of 16 rows of one chunk), V with f(r) = 2 (r & 7), whose transposing
+  // reads (below) then hit 16 distinct slots per half wave. Rows past kv_end
+  // repeat key kv_end - 1: K's scores there are masked to -inf, so whatever P
+  // (0) multiplies in V is finite.
+  constexpr int NB = HW == 2 ? 4 : 2;
+  uint16_t *k_lds0 = pf_lds;                  // [NB][64 keys][128] swizzled
+  uint16_t *v_lds0 = pf_lds + NB * PKB * D;   // [NB][64 keys][128] swizzled
+  // (16 instructions of 4 rows a block each, spread over the waves: a wave's
+  // rows are 16 HW apart, so their swizzle is one value per lane)
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  const int drow = 4 * wv + (lane >> 4);
+  const uint32_t kx = (uint32_t)((lane & 15) ^ (drow & 15)) << 4;
+  const uint32_t vx = (uint32_t)((lane & 15) ^ (2 * (drow & 7))) << 4;
+  auto dma_k = [&](int blk) {
+    const uint32_t dst = lds_u32(k_lds0 + (blk & (NB - 1)) * PKB * D) + 1024 * wv;
+#pragma unroll
+    for (int n = 0; n < 4 / HW; ++n) {
+      const int key = min(blk * PKB + drow + 16 * HW * n, kv_end - 1);
+      lds_dma16_asm(a.kc + kv_base, (uint32_t)key * (2 * D) + kx, dst + 4096 * HW * n);
+    }
+  };
+  auto dma_v = [&](int blk) {
+    const uint32_t dst = lds_u32(v_lds0 + (blk & (NB - 1)) * PKB * D) + 1024 * wv;
+#pragma unroll
+    for (int n = 0; n < 4 / HW; ++n) {
+      const int key = min(blk * PKB + drow + 16 * HW * n, kv_end - 1);
+      lds_dma16_asm(a.vc + kv_base, (uint32_t)key * (2 * D) + vx, dst + 4096 * HW * n);
+    }
+  };
+  // the first copies go out before anything else (q's loads overlap them)
+  // K blocks 0 .. NB - 1, V blocks 0 .. NB - 2
+  for (int j = 0; j < NB; ++j) {
+    if (j < nblk) dma_k(j);
+    if (j < nblk && j < NB - 1) dma_v(j);
+  }
 
-  // q^T fragments: lane (row col of tile r, dims 32 t + 8 g4 ..), bf16 hi + lo
-  // of c q in f32, so the scores come out as c s (c = scale * log2(e))
-  u32x4 qhi[R][4], qlo[R][4];
+  // p = exp(scale s - m) = exp2(c s - m'), c = scale * log2(e) > 0. (Below
+  // 1e-30 every visible key weighs the same either way; a masked key's c (-inf)
+  // has to stay -inf.)
+  const float cs = a.scale * 1.4426950408889634f;
+  const float c = cs < 1e-30f ? 1e-30f : cs;
+
+  // q^T fragments: lane (row col of tile r, dims 32 t + 8 g4 ..). A bf16 q is
+  // the operand as it is; an f32 q (LO) takes bf16 hi + lo parts.
+  u32x4 qhi[R][4], qlo[LO ? R : 1][4];
+  // (every load goes out before the first conversion waits for one)
+  const int64_t q_off = (int64_t)b * a.q_sb + (int64_t)hq * a.q_sh + 8 * g4;
+  int64_t q_row[R];
 #pragma unroll
-  for (int r = 0; r < R; ++r)
+  for (int r = 0; r < R; ++r) q_row[r] = q_off + (int64_t)min(i0 + 16 * r + col, a.S - 1) * a.q_ss;
+  if constexpr (LO) {
+    f32x4 raw[R][4][2];
 #pragma unroll
-    for (int t = 0; t < 4; ++t) {
-      const int my_i = min(i0 + 16 * r + col, a.S - 1);
-      const int64_t off = (int64_t)b * a.q_sb + (int64_t)my_i * a.q_ss + (int64_t)hq * a.q_sh + 32 * t + 8 * g4;
-      float v[8];
-      if (a.q_f32) {
-        const f32x4 lo = *(const f32x4 *)((const float *)a.q + off);
-        const f32x4 hi = *(const f32x4 *)((const float *)a.q + off + 4);
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) raw[r][t][e] = *(const f32x4 *)((const float *)a.q + q_row[r] + 32 * t + 4 * e);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          v[e] = lo[e];
-          v[4 + e] = hi[e];
+          const float v0 = raw[r][t][e >> 1][2 * (e & 1)], v1 = raw[r][t][e >> 1][2 * (e & 1) + 1];
+          const float h0 = round_bf16(v0), h1 = round_bf16(v1);
+          qhi[r][t][e] = pack_bf16x2(h0, h1);
+          qlo[r][t][e] = pack_bf16x2(v0 - h0, v1 - h1);
         }
-      } else {
-        unpack_bf16x8(*(const u32x4 *)((const uint16_t *)a.q + off), v);
-      }
+  } else {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] *= c_exp;
+    for (int r = 0; r < R; ++r)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float h0 = round_bf16(v[2 * e]), h1 = round_bf16(v[2 * e + 1]);
-        qhi[r][t][e] = pack_bf16x2(h0, h1);
-        qlo[r][t][e] = pack_bf16x2(v[2 * e] - h0, v[2 * e + 1] - h1);
-      }
-    }
+      for (int t = 0; t < 4; ++t) qhi[r][t] = *(const u32x4 *)((const uint16_t *)a.q + q_row[r] + 32 * t);
+  }
 
   f32x4 o[R][8];
   float m_run[R], l_run[R];
@@ -1231,34 +1296,6 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
     for (int dt = 0; dt < 8; ++dt) o[r][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
 
-  // Block staging by LDS DMA (no registers held across the block), both
-  // operands double-buffered and row-major with 16-byte chunks XOR-swizzled
-  // by row (the lane writing LDS chunk slot c' of row r fetches global chunk
-  // c' ^ f(r)): K with f(r) = r & 15 (conflict-free fragment reads of 16 rows
-  // of one chunk), V with f(r) = 2 (r & 7), whose transposing reads (below)
-  // then hit 16 distinct slots per half wave. K rows past kv_end are not
-  // copied (their scores are masked to -inf); V rows past kv_end repeat key
-  // kv_end - 1, so whatever P multiplies there is finite (and P is 0).
-  uint16_t *k_lds0 = pf_lds;                 // [2][64 keys][128] swizzled
-  uint16_t *v_lds0 = pf_lds + 2 * PKB * D;   // [2][64 keys][128] swizzled
-  auto dma_block = [&](int blk) {
-    uint16_t *kb = k_lds0 + (blk & 1) * PKB * D;
-    uint16_t *vb = v_lds0 + (blk & 1) * PKB * D;
-    // 2 x 16 instructions of 64 lanes (K, then V), spread over the waves
-    for (int ins = __builtin_amdgcn_readfirstlane(wave); ins < 32; ins += 4 * HW) {
-      const int gidx = 64 * (ins & 15) + lane;  // 16-byte granule of the block
-      const int r = gidx >> 4, c = gidx & 15;
-      const int key = blk * PKB + r;
-      if (ins < 16) {
-        if (key < kv_end)
-          lds_dma16_asm(a.kc + kv_base, (uint32_t)(key * D + ((c ^ (r & 15)) << 3)) * 2u,
-                        lds_u32(kb + 64 * 8 * (ins & 15)));
-      } else {
-        lds_dma16_asm(a.vc + kv_base, (uint32_t)(min(key, kv_end - 1) * D + ((c ^ (2 * (r & 7))) << 3)) * 2u,
-                      lds_u32(vb + 64 * 8 * (ins & 15)));
-      }
-    }
-  };
   // The V^T operand of O^T += V^T P^T straight from row-major V by
   // ds_read_b64_tr_b16: in each 16-lane group, lane 4j + q reads the 4
   // values d0 + 4q .. + 3 of key row k_j, and lane i receives the values at
@@ -1266,17 +1303,22 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
   // 32 ks + 4 g4 + 0..3 and 32 ks + 16 + 4 g4 + 0..3 (the key order of its P
   // operand) at d = 16 dt + col: two reads.
   const int tr_j = col >> 2, tr_q = col & 3;
-  auto v_frag = [&](const uint16_t *vb, int ks, int dt) {
+  // LDS byte addresses of the fragments: one XOR and a constant offset from
+  // these (chunk 4 t + g4 of K row col, values 16 dt + 4 tr_q of V row 4 g4 + tr_j)
+  uint32_t k_frag0 = lds_u32(k_lds0) + 2 * col * D + ((g4 ^ col) << 4);
+  uint32_t v_frag0 = lds_u32(v_lds0) + 2 * (4 * g4 + tr_j) * D +
+                     ((2 * ((4 * g4 + tr_j) & 7)) << 4) + ((tr_q & 1) << 3);
+  v_frag0 ^= (tr_q >> 1) << 4;
+  auto k_frag = [&](uint32_t base, int kt, int t) {
+    return *(const __attribute__((address_space(3))) u32x4 *)(uintptr_t)((base ^ (t << 6)) + 2 * 16 * kt * D);
+  };
+  auto v_frag = [&](uint32_t base, int ks, int dt) {
     u32x4 va;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int row = 32 * ks + 16 * h + 4 * g4 + tr_j;
-      const int d0 = 16 * dt + 4 * tr_q;
-      const int slot = (d0 >> 3) ^ (2 * (row & 7));
-      const uint16_t *src = vb + row * D + slot * 8 + (d0 & 7);
       typedef short v4i16 __attribute__((ext_vector_type(4)));
       const v4i16 t = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-          (__attribute__((address_space(3))) v4i16 *)(src));
+          (__attribute__((address_space(3))) v4i16 *)(uintptr_t)((base ^ (dt << 5)) + 2 * (32 * ks + 16 * h) * D));
       const uint2 u = __builtin_bit_cast(uint2, t);
       va[2 * h] = u.x;
       va[2 * h + 1] = u.y;
@@ -1284,102 +1326,188 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
     return va;
   };
 
-  dma_block(0);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  for (int blk = 0; blk < nblk; ++blk) {
-    const uint16_t *ks_lds = k_lds0 + (blk & 1) * PKB * D;
-    const uint16_t *vs_lds = v_lds0 + (blk & 1) * PKB * D;
-    if (blk + 1 < nblk) dma_block(blk + 1);  // in flight while this block is used
-    const int j0 = blk * PKB;
-    if (j0 <= wave_last) {  // wave-uniform: else every key of the block is in this wave's future
-      // S^T tiles: s[r][kt] lane (key j0 + 16 kt + 4 g4 + i, row col of tile r)
-      f32x4 s[R][4];
+  // (wave-uniform, as scalars)
+  const int ph = HW == 2 ? __builtin_amdgcn_readfirstlane(head) : 0;
+  // blocks this wave's rows see (none: every row past the end)
+  const int nact = __builtin_amdgcn_readfirstlane(i0 < a.S ? wave_last / PKB + 1 : 0);
+  f32x4 s[R][4];
+  u32x4 pb[R][2];
+  // Matrix half: PV of block blk - 1, then QK of block blk, 16 fragments each,
+  // the LDS reads NF - 1 fragments ahead of their MFMAs.
+  constexpr int NF = 5;
+  auto matrix_half = [&](int blk, auto pv, auto qk) {
+    constexpr int N0 = decltype(pv)::value ? 0 : 16, N1 = decltype(qk)::value ? 32 : 16;
+    uint32_t vs = v_frag0 + ((blk - 1) & (NB - 1)) * (2 * PKB * D), ks0 = k_frag0 + (blk & (NB - 1)) * (2 * PKB * D);
+    asm("" : "+v"(vs), "+v"(ks0));  // (the per-fragment XORs stay in the loop, not in registers)
+    u32x4 fr[NF];
+    auto read = [&](int n) {
+      fr[n % NF] = n < 16 ? v_frag(vs, n >> 3, n & 7) : k_frag(ks0, 2 * ((n - 16) >> 3) + (n & 1), (n >> 1) & 3);
+    };
 #pragma unroll
-      for (int kt = 0; kt < 4; ++kt) {
-        const int kr = kt * 16 + col;
-        f32x4 acc[R];
+    for (int n = N0; n < N0 + NF - 1; ++n) read(n);
 #pragma unroll
-        for (int r = 0; r < R; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int n = N0; n < N1; ++n) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (n + NF - 1 < N1) read(n + NF - 1);
+      __builtin_amdgcn_sched_barrier(0);
+      const bf16x8 f = as_bf16x8(fr[n % NF]);
+      if (n < 16) {
+        // O^T += V^T P^T: the V^T operand in the key order of pb
 #pragma unroll
-        for (int t = 0; t < 4; ++t) {
-          const u32x4 kf = *(const u32x4 *)(ks_lds + kr * D + (((4 * t + g4) ^ col) << 3));
+        for (int r = 0; r < R; ++r) o[r][n & 7] = mfma16x16x32(f, as_bf16x8(pb[r][(n >> 3) & 1]), o[r][n & 7]);
+      } else {
+        // S^T tiles: s[r][kt] lane (key 64 blk + 16 kt + 4 g4 + i, row col of tile r)
+        // (key tiles in pairs, so 2 R accumulators take turns)
+        const int t = (n >> 1) & 3, kt = (2 * ((n - 16) >> 3) + (n & 1)) & 3;
 #pragma unroll
-          for (int r = 0; r < R; ++r) {
-            acc[r] = mfma16x16x32(as_bf16x8(kf), as_bf16x8(qhi[r][t]), acc[r]);
-            acc[r] = mfma16x16x32(as_bf16x8(kf), as_bf16x8(qlo[r][t]), acc[r]);
-          }
+        for (int r = 0; r < R; ++r) {
+          if (t == 0) s[r][kt] = f32x4{0.f, 0.f, 0.f, 0.f};
+          s[r][kt] = mfma16x16x32(f, as_bf16x8(qhi[r][t]), s[r][kt]);
         }
+        if constexpr (LO)
 #pragma unroll
-        for (int r = 0; r < R; ++r) s[r][kt] = acc[r];
+          for (int r = 0; r < R; ++r) s[r][kt] = mfma16x16x32(f, as_bf16x8(qlo[r][t]), s[r][kt]);
       }
-      u32x4 pb[R][2];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // p = exp2(c s - m) of tile r, l's part of it, and P as the MFMA operand.
+  auto weights = [&](int r, auto exponent) {
+    float ls[2] = {0.f, 0.f};
+    float e[4][4];
+#pragma unroll
+    for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        // (v_exp_f32: terms below 2^-126 of the reference m flush to zero)
+        e[kt][i] = __builtin_amdgcn_exp2f(exponent(s[r][kt][i]));
+        ls[i & 1] += e[kt][i];
+      }
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+      pb[r][ks] = u32x4{pack_bf16x2(e[2 * ks][0], e[2 * ks][1]), pack_bf16x2(e[2 * ks][2], e[2 * ks][3]),
+                        pack_bf16x2(e[2 * ks + 1][0], e[2 * ks + 1][1]),
+                        pack_bf16x2(e[2 * ks + 1][2], e[2 * ks + 1][3])};
+    return ls[0] + ls[1];
+  };
+  // Vector half: the softmax of block blk. The reference m is not every
+  // block's maximum: it stays while each lane's 16 weights sum to at most 2^8,
+  // so p <= 2^8 (exact in bf16's range; l and O carry the same factor and
+  // O / l is unchanged). Most blocks then take no maximum and rescale nothing;
+  // where a sum exceeds that (block 0: m = -inf) the block's maxima become m
+  // and its weights are formed again. Key 0 is visible to every row and block
+  // 0 is never skipped, so m is finite from there on.
+  auto vector_half = [&](int blk) {
+    const int j0 = blk * PKB;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      // the causal mask only where some key of the block lies past the
+      // tile's first row (wave-uniform)
+      if (j0 + PKB - 1 > start + i0 + 16 * r) {
+        const int last = my_pos[r] - j0 - 4 * g4;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (16 * kt + i > last) s[r][kt][i] = kNegInf;
+      }
+    }
+    float ls[R];
+    bool moves = false;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      ls[r] = weights(r, [&](float v) { return fmaf(v, c, -m_run[r]); });
+      moves |= !(ls[r] <= 256.f);
+    }
+    if (__ballot(moves)) {
+#pragma clang fp contract(off)
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        // Scores c s (the scale and log2(e) are folded into q); the causal
-        // mask only where some key of the block lies past the tile's first
-        // row (wave-uniform).
-        if (j0 + PKB - 1 > start + i0 + 16 * r) {
-#pragma unroll
-          for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              if (j0 + 16 * kt + 4 * g4 + i > my_pos[r]) s[r][kt][i] = kNegInf;
-        }
         float mb = kNegInf;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
           for (int i = 0; i < 4; ++i) mb = fmaxf(mb, s[r][kt][i]);
-        mb = wave_max4(mb);
-        // key 0 is visible to every row and block 0 is never skipped, so
-        // m_new is finite from the first block on (f = exp2(-inf) = 0 there).
-        // p = exp(scale (s - m)) = exp2(c s - c m) on v_exp_f32 (terms below
-        // 2^-126 of the reference flush to zero). The reference m moves only
-        // when a block's maximum exceeds it by more than 8 (log2 units), so
-        // p <= 2^8 (exact in bf16's range; l and O carry the same factor and
-        // O / l is unchanged) and most blocks rescale nothing
-        const float m_new = mb > m_run[r] + 8.f ? mb : m_run[r];
+        // (a sum past 2^8 has a weight past 2^4; c s rounded by itself, not
+        // within an fma: the largest score's p is then exactly 1)
+        const float mx = wave_max4(mb) * c;
+        const float m_new = mx > m_run[r] + 4.f ? mx : m_run[r];
         const float f = __builtin_amdgcn_exp2f(m_run[r] - m_new);
-        float ls = 0.f;
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float e = __builtin_amdgcn_exp2f(s[r][kt][i] - m_new);
-            s[r][kt][i] = e;
-            ls += e;
-          }
-        l_run[r] = l_run[r] * f + wave_sum4(ls);
+        l_run[r] *= f;
         m_run[r] = m_new;
-        if (__ballot(f != 1.f))  // no row's maximum moved: nothing to rescale
 #pragma unroll
-          for (int dt = 0; dt < 8; ++dt) o[r][dt] *= f;
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-          pb[r][ks] = u32x4{pack_bf16x2(s[r][2 * ks][0], s[r][2 * ks][1]),
-                            pack_bf16x2(s[r][2 * ks][2], s[r][2 * ks][3]),
-                            pack_bf16x2(s[r][2 * ks + 1][0], s[r][2 * ks + 1][1]),
-                            pack_bf16x2(s[r][2 * ks + 1][2], s[r][2 * ks + 1][3])};
+        for (int dt = 0; dt < 8; ++dt) o[r][dt] *= f;
+        ls[r] = weights(r, [&](float v) {
+#pragma clang fp contract(off)
+          return v * c - m_run[r];
+        });
       }
-      // O^T += V^T P^T: the V^T operand in the key order of pb
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-        for (int dt = 0; dt < 8; ++dt) {
-          const u32x4 va = v_frag(vs_lds, ks, dt);
-#pragma unroll
-          for (int r = 0; r < R; ++r) o[r][dt] = mfma16x16x32(as_bf16x8(va), as_bf16x8(pb[r][ks]), o[r][dt]);
-        }
     }
-    // the next block's copies are in; every wave is done with this block
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < R; ++r) l_run[r] += ls[r];
+    // (computed here: the compiler would sink the exponentials to their use
+    // in the matrix half, past the barrier)
+#pragma unroll
+    for (int r = 0; r < R; ++r) asm volatile("" : "+v"(pb[r][0]), "+v"(pb[r][1]), "+v"(l_run[r]));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Step j's copies (j > 0): K block j + NB - 1 and V block j + NB - 2, issued
+  // by every wave once both heads are done with matrix half j - 1, whose slots
+  // they take.
+  auto dma_step = [&](int j) {
+    if (j + NB - 1 < nblk) dma_k(j + NB - 1);
+    if (j + NB - 2 < nblk) dma_v(j + NB - 2);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // barrier; before it this wave's LDS reads are done and, with landed, its
+  // copies of K block j + 1 and V block j are in (those of the NB - 2 steps
+  // up to j may be in flight: 8 / HW instructions a step)
+  auto sync = [&](bool landed, int j) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (landed) {
+      if (NB == 4 && j + NB - 1 < nblk) asm volatile("s_waitcnt vmcnt(8) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    } else {
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  static_assert(HW == 1 || (NB == 4 && 8 / HW * (NB - 2) == 8), "the wait's count");
+
+  sync(true, nblk);
+  if (ph) sync(false, 0);  // the second head's waves run half a step later
+  auto to_vector = [&](int blk) {
+    if (HW == 2) sync(ph, blk);
+    if (ph) dma_step(blk + 1);
+  };
+  auto to_matrix = [&](int blk) {
+    sync(!ph, blk);
+    if (!ph) dma_step(blk + 1);
+  };
+  int blk = 0;
+  if (nact > 0) {
+    matrix_half(0, No{}, Yes{});
+    for (; blk + 1 < nact; ++blk) {
+      to_vector(blk);
+      vector_half(blk);
+      to_matrix(blk);
+      matrix_half(blk + 1, Yes{}, Yes{});
+    }
+    to_vector(blk);
+    vector_half(blk);
+    to_matrix(blk);
+    matrix_half(blk + 1, Yes{}, No{});
+    ++blk;
   }
+  for (; blk < nblk; ++blk) {  // blocks past this wave's rows
+    to_vector(blk);
+    to_matrix(blk);
+  }
+  if (HW == 2 && !ph) sync(false, 0);  // (the second head's last vector half)
 #pragma unroll
   for (int r = 0; r < R; ++r) {
+    const float inv = 1.0f / wave_sum4(l_run[r]);
     if (i0 + 16 * r + col >= a.S) continue;
-    const float inv = 1.0f / l_run[r];
     const int64_t ob = (int64_t)b * a.o_sb + (int64_t)(i0 + 16 * r + col) * a.o_ss + (int64_t)hq * a.o_sh;
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
@@ -1403,7 +1531,11 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
   }                                                                                  \
   extern "C" __global__ void __launch_bounds__(256 * (G < 2 ? G : 2))                \
       __attribute__((amdgpu_waves_per_eu(2))) rxw8_gqa_prefill_r2_d128_g##G(PrefillArgs a) { \
-    attn_prefill_rt<G, 2>(a);                                                        \
+    attn_prefill_rt<G, 2, false>(a);                                                 \
+  }                                                                                  \
+  extern "C" __global__ void __launch_bounds__(256 * (G < 2 ? G : 2))                \
+      __attribute__((amdgpu_waves_per_eu(2))) rxw8_gqa_prefill_r2q32_d128_g##G(PrefillArgs a) { \
+    attn_prefill_rt<G, 2, true>(a);                                                  \
   }
 RXW8_PREFILL(1)
 RXW8_PREFILL(2)
@@ -1412,7 +1544,11 @@ RXW8_PREFILL(4)
 // two heads per kv head)
 extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
 rxw8_gqa_prefill_r2_d128_g8(PrefillArgs a) {
-  attn_prefill_rt<8, 2>(a);
+  attn_prefill_rt<8, 2, false>(a);
+}
+extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))
+rxw8_gqa_prefill_r2q32_d128_g8(PrefillArgs a) {
+  attn_prefill_rt<8, 2, true>(a);
 }
 
 // ---- generic decode attention (any D <= 256, any group, f32 or bf16 cache):

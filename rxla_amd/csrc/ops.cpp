@@ -1573,10 +1573,12 @@ int prefill_launch(Runtime *rt, const void *q, int q_f32, int64_t q_sb, int64_t 
   // The two-tile kernel: one query head per wave, min(G, 2) heads per
   // workgroup (4 waves each; G = 4 takes two workgroups per kv head), two
   // 16-row tiles per wave (128 query rows per workgroup), K and V by LDS
-  // DMA: at the C5 prompt shape 72.8 us against 94.3 (one tile) and 120.5
-  // (all heads per wave, one wave per SIMD). RXW8_PREFILL_R2=0 selects the
-  // one-tile kernel for G <= 2 and the all-heads one for G = 4;
-  // RXW8_PREFILL_R2=0 RXW8_PREFILL_WH=0 the all-heads one for every G.
+  // DMA, the two heads half a step apart: at 4 x 2048 rows, 32 heads, 170 us
+  // against 220 for the same tiles in step; at the C5 prompt shape (already
+  // with the tiles in step) 72.8 against 94.3 (one tile) and 120.5 (all heads
+  // per wave, one wave per SIMD). RXW8_PREFILL_R2=0 selects the one-tile
+  // kernel for G <= 2 and the all-heads one for G = 4; RXW8_PREFILL_R2=0
+  // RXW8_PREFILL_WH=0 the all-heads one for every G.
   static const int wh_env = env_int("RXW8_PREFILL_WH", 1);
   static const int r2_env = env_int("RXW8_PREFILL_R2", 1);
   // (the two-tile kernel addresses a cache plane with 32-bit byte offsets)
@@ -1591,7 +1593,7 @@ int prefill_launch(Runtime *rt, const void *q, int q_f32, int64_t q_sb, int64_t 
   }
   if (r2) a.nqb = (int)((S + 127) / 128);
   std::snprintf(kname, sizeof kname,
-                r2 ? "rxw8_gqa_prefill_r2_d128_g%d"
+                r2 ? (q_f32 ? "rxw8_gqa_prefill_r2q32_d128_g%d" : "rxw8_gqa_prefill_r2_d128_g%d")
                    : (wh ? "rxw8_gqa_prefill_wh_d128_g%d" : "rxw8_gqa_prefill_d128_g%d"),
                 G);
   // K and V^T blocks of 64 keys, double-buffered (2 x (64*128 + 128*72) bf16)
@@ -1599,7 +1601,9 @@ int prefill_launch(Runtime *rt, const void *q, int q_f32, int64_t q_sb, int64_t 
   // the two-tile kernel: min(G, 2) heads per workgroup, G / min(G, 2) workgroups per kv head
   const int hw = G < 2 ? G : 2;
   if (r2)
-    return launch(rt, kname, dim3((unsigned)(a.nqb * B * Hkv * (G / hw))), dim3(256 * hw), a, lds);
+    // rings of 4 (2 for one head per workgroup) K and V blocks of 64 keys
+    return launch(rt, kname, dim3((unsigned)(a.nqb * B * Hkv * (G / hw))), dim3(256 * hw), a,
+                  (size_t)2 * 2 * hw * 64 * 128 * 2);
   return launch(rt, kname, dim3((unsigned)(a.nqb * B * Hkv)), dim3(wh ? 256 * G : 256), a, lds);
 }
 
