@@ -893,14 +893,25 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
 
-// One chunk of one (sequence, head): 256 threads (4 waves).
+// One chunk of one (sequence, head): 512 threads (8 waves). The solve goes by
+// 16-row blocks on the matrix cores,
+//   X_i = D_i (B_i - sum_{j<i} A_ij X_j),  D_i = (I + A_ii)^-1,
+// 16 columns of X = [U | W] per tile, DL / 64 tiles per wave: row 4 (l / 16) + r
+// of a product's lane l is the k index step r of the next product asks of the
+// same lane, so X passes from one to the next in registers; only the four
+// 16 x 16 D_i are substituted out (wave 0, a column per lane, under the other
+// waves' Q K^T). At 500 positions, 16 heads of 128 (128 workgroups, half the
+// CUs): 32.5 -> 17 us against one thread per column of X for all 64 rows (2016
+// dependent multiply-adds and as many LDS reads). Serial chains bound it: the
+// load, three products one after another, a barrier between each.
 template <int DL>
 __device__ void delta_chunk(const Q35ChunkArgs &a) {
-  constexpr int C = 64, KP = DL + 4, KQ = DL / 4;
+  constexpr int C = 64, KP = DL + 4, KQ = DL / 4, CT = DL / 16, NT = 2 * CT / 8;
   __shared__ __attribute__((aligned(16))) float ks[C][KP], qs[C][KP];
-  __shared__ __attribute__((aligned(16))) float as[C][C + 4];
+  __shared__ __attribute__((aligned(16))) float as[C][C + 4];      // -A below the diagonal
+  __shared__ __attribute__((aligned(16))) float dinv[4][16][20];
   __shared__ float bs[C], gs[C];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g = lane >> 4;
   const int64_t ch = blockIdx.x;
   const int bh = (int)(ch / a.NC), c = (int)(ch - (int64_t)bh * a.NC);
@@ -908,44 +919,121 @@ __device__ void delta_chunk(const Q35ChunkArgs &a) {
   const int t0 = c * C, n = min(C, a.S - t0);
   const int64_t W = (int64_t)a.Hl * DL;
   const int64_t row0 = (int64_t)b * a.S + t0;
-  // the v column of the U half of the solve, loaded first (thread = column)
-  float x[C];
+  // beta and the log decays, then k and q rows of the chunk (rows past the
+  // sequence zero), and the v values of this wave's U tiles in the products'
+  // layout: every load out before the first is waited for
+  const int64_t brow = (row0 + min(lane, n - 1)) * a.Hl + h;
+  float lg = wave == 0 ? a.lg[brow] : 0.f, bt = wave == 0 ? a.beta[brow] : 0.f;
+  f32x4 qv[KQ / 8], kv[KQ / 8];
 #pragma unroll
-  for (int t = 0; t < C; ++t)
-    x[t] = tid < DL && t < n ? a.mixed[(row0 + t) * 3 * W + 2 * W + (int64_t)h * DL + tid] : 0.f;
-  // k and q rows of the chunk (rows past the sequence zero)
-  for (int e = tid; e < C * KQ; e += 256) {
-    const int t = e / KQ, d4 = e - t * KQ;
-    float4 qv = {0.f, 0.f, 0.f, 0.f}, kv = qv;
-    if (t < n) {
-      const float *m = a.mixed + (row0 + t) * 3 * W + (int64_t)h * DL + 4 * d4;
-      qv = *(const float4 *)m;
-      kv = *(const float4 *)(m + W);
-    }
-    *(float4 *)&qs[t][4 * d4] = qv;
-    *(float4 *)&ks[t][4 * d4] = kv;
+  for (int e = 0; e < KQ / 8; ++e) {
+    const int t = (tid + 512 * e) / KQ, d4 = (tid + 512 * e) % KQ;
+    const float *m = a.mixed + (row0 + min(t, n - 1)) * 3 * W + (int64_t)h * DL + 4 * d4;
+    qv[e] = *(const f32x4 *)m;
+    kv[e] = *(const f32x4 *)(m + W);
   }
-  if (wave == 0) {  // inclusive scan of the log decays; beta
-    float x = lane < n ? a.lg[(row0 + lane) * a.Hl + h] : 0.f;
+  float x[NT][4][4];  // tile j of this wave: column tile (wave + 8 j) of [U | W], rows 16 i + 4 g + r
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    if (wave + 8 * j < CT)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          x[j][i][r] = a.mixed[(row0 + min(16 * i + 4 * g + r, n - 1)) * 3 * W + 2 * W + (int64_t)h * DL +
+                               16 * (wave + 8 * j) + r16];
+  __builtin_amdgcn_sched_barrier(0);
+  if (wave == 0) {  // inclusive scan of the log decays; beta (0 past the sequence)
+    if (lane >= n) lg = bt = 0.f;
+#pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const float y = __shfl_up(x, o);
-      if (lane >= o) x += y;
+      const float y = __shfl_up(lg, o);
+      if (lane >= o) lg += y;
     }
-    gs[lane] = x;
-    bs[lane] = lane < n ? a.beta[(row0 + lane) * a.Hl + h] : 0.f;
+    gs[lane] = lg;
+    bs[lane] = bt;
+  }
+#pragma unroll
+  for (int e = 0; e < KQ / 8; ++e) {
+    const int t = (tid + 512 * e) / KQ, d4 = (tid + 512 * e) % KQ;
+    *(f32x4 *)&qs[t][4 * d4] = t < n ? qv[e] : f32x4{0.f, 0.f, 0.f, 0.f};
+    *(f32x4 *)&ks[t][4 * d4] = t < n ? kv[e] : f32x4{0.f, 0.f, 0.f, 0.f};
   }
   __syncthreads();
+  // Row tile i against column tile j of rows x K^T (the MFMA k index of lane l
+  // at step 4 q + e is 16 q + 4 (l / 16) + e in both operands: 16-byte reads)
+  auto product = [&](const float (*rows)[KP], int i, int j) {
+    f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int q = 0; q < KQ / 4; ++q) {
+      const float4 u = *(const float4 *)&rows[16 * i + r16][16 * q + 4 * g];
+      const float4 k = *(const float4 *)&ks[16 * j + r16][16 * q + 4 * g];
+      acc[0] = mfma4(u.x, k.x, acc[0]);
+      acc[1] = mfma4(u.y, k.y, acc[1]);
+      acc[0] = mfma4(u.z, k.z, acc[0]);
+      acc[1] = mfma4(u.w, k.w, acc[1]);
+    }
+    return acc[0] + acc[1];
+  };
+  // tile index t of the 10 on and below the diagonal -> (i, j)
+  auto tile_row = [](int t) { return t < 1 ? 0 : t < 3 ? 1 : t < 6 ? 2 : 3; };
+  for (int t = wave; t < 10; t += 8) {
+    const int i = tile_row(t), j = t - i * (i + 1) / 2;
+    const f32x4 kk = product(ks, i, j);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int p = 16 * i + 4 * g + r, s2 = 16 * j + r16;
+      // (gam is non-increasing, so the exponent is <= 0 wherever s <= t)
+      as[p][s2] = s2 < p ? -(bs[p] * expf(fminf(gs[p] - gs[s2], 0.f)) * kk[r]) : 0.f;
+    }
+  }
+  __syncthreads();
+  float *pm = a.pm + ch * C * C;
+  if (wave == 0) {  // D_g, column r16
+    float d[16];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+      float p0 = t == r16 ? 1.f : 0.f, p1 = 0.f, p2 = 0.f, p3 = 0.f;
+#pragma unroll
+      for (int s2 = 0; s2 < t; s2 += 4) {
+        const float4 a4 = *(const float4 *)&as[16 * g + t][16 * g + s2];
+        p0 += a4.x * d[s2];
+        if (s2 + 1 < t) p1 += a4.y * d[s2 + 1];
+        if (s2 + 2 < t) p2 += a4.z * d[s2 + 2];
+        if (s2 + 3 < t) p3 += a4.w * d[s2 + 3];
+      }
+      d[t] = (p0 + p1) + (p2 + p3);
+      dinv[g][t][r16] = d[t];
+    }
+  } else {
+    for (int t = wave - 1; t < 10; t += 7) {
+      const int i = tile_row(t), j = t - i * (i + 1) / 2;
+      const f32x4 qk = product(qs, i, j);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int p = 16 * i + 4 * g + r, s2 = 16 * j + r16;
+        pm[p * C + s2] = s2 <= p ? expf(fminf(gs[p] - gs[s2], 0.f)) * qk[r] : 0.f;
+      }
+    }
+    if (wave >= 2) {  // the 6 tiles above the diagonal
+      const int t = wave - 2, i = t < 3 ? 0 : t < 5 ? 1 : 2, j = t < 3 ? t + 1 : t < 5 ? t - 1 : 3;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) pm[(16 * i + 4 * g + r) * C + 16 * j + r16] = 0.f;
+    }
+  }
   // Qg = diag(Gamma) Q; KdT[i][s] = (Gamma_end / Gamma_s) k_s[i]
   {
     float *qg = a.qg + ch * C * DL, *kdt = a.kdt + ch * C * DL;
     const float gend = gs[C - 1];
-    for (int e = tid; e < C * KQ; e += 256) {
+#pragma unroll
+    for (int e = tid; e < C * KQ; e += 512) {
       const int t = e / KQ, d4 = e - t * KQ;
       const float f = expf(gs[t]);
       const float4 q4 = *(const float4 *)&qs[t][4 * d4];
       *(float4 *)(qg + t * DL + 4 * d4) = float4{f * q4.x, f * q4.y, f * q4.z, f * q4.w};
     }
-    for (int e = tid; e < DL * (C / 4); e += 256) {
+#pragma unroll
+    for (int e = tid; e < DL * (C / 4); e += 512) {
       const int i = e / (C / 4), s4 = 4 * (e - i * (C / 4));
       float4 o;
       o.x = expf(gend - gs[s4]) * ks[s4][i];
@@ -955,209 +1043,227 @@ __device__ void delta_chunk(const Q35ChunkArgs &a) {
       *(float4 *)(kdt + i * C + s4) = o;
     }
   }
-  // K K^T and Q K^T, row tile = wave, column tiles 0..3; the MFMA k index of
-  // lane l at step kk is 4 kk + l / 16 (the same in both operands; rows 132
-  // floats apart put a step's 64 reads on distinct banks two by two)
-  f32x4 kk_acc[4], qk_acc[4];
+  // B: beta_t v_t (U), beta_t Gamma_t k_t (W); rows past the sequence zero
 #pragma unroll
-  for (int j = 0; j < 4; ++j) kk_acc[j] = qk_acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int kk = 0; kk < KQ; ++kk) {
-    const int d = 4 * kk + g;
-    const float ak = ks[16 * wave + r16][d], aq = qs[16 * wave + r16][d];
+  for (int j = 0; j < NT; ++j) {
+    const bool is_w = wave + 8 * j >= CT;
+    const int col = 16 * (wave + 8 * j - (is_w ? CT : 0)) + r16;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float bk = ks[16 * j + r16][d];
-      kk_acc[j] = mfma4(ak, bk, kk_acc[j]);
-      qk_acc[j] = mfma4(aq, bk, qk_acc[j]);
-    }
-  }
-  // lane holds rows t = 16 wave + 4 g + r, columns s = 16 j + r16
-  float *pm = a.pm + ch * C * C;
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = 16 * wave + 4 * g + r, s2 = 16 * j + r16;
-      // (gam is non-increasing, so the exponent is <= 0 wherever s <= t)
-      const float e = expf(fminf(gs[t] - gs[s2], 0.f));
-      as[t][s2] = s2 < t ? bs[t] * e * kk_acc[j][r] : 0.f;
-      pm[t * C + s2] = s2 <= t ? e * qk_acc[j][r] : 0.f;
-    }
-  __syncthreads();
-  // forward substitution, thread = one column of X = [U | W]:
-  //   X_t = B_t - sum_{s<t} A_ts X_s,  B_t = beta_t v_t (U), beta_t Gamma_t k_t (W)
-  if (tid < 2 * DL) {
-    const bool is_w = tid >= DL;
-    const int col = is_w ? tid - DL : tid;
-#pragma unroll
-    for (int t = 0; t < C; ++t) x[t] = (is_w ? bs[t] * expf(gs[t]) * ks[t][col] : bs[t] * x[t]);
-    // row t's A values are read while row t - 1 is reduced (one LDS round
-    // trip per row, not one per pair of reads)
-    float4 arow[2][C / 4];
-    arow[1][0] = *(const float4 *)&as[1][0];
-#pragma unroll
-    for (int t = 1; t < C; ++t) {
-      const int cur = t & 1;
-      if (t + 1 < C)
-#pragma unroll
-        for (int q = 0; q < (t + 4) / 4; ++q) arow[cur ^ 1][q] = *(const float4 *)&as[t + 1][4 * q];
-      float p0 = 0.f, p1 = 0.f, p2 = 0.f, p3 = 0.f;
-#pragma unroll
-      for (int s2 = 0; s2 < t; s2 += 4) {  // A_ts = 0 for s >= t
-        const float4 a4 = arow[cur][s2 / 4];
-        p0 += a4.x * x[s2];
-        if (s2 + 1 < t) p1 += a4.y * x[s2 + 1];
-        if (s2 + 2 < t) p2 += a4.z * x[s2 + 2];
-        if (s2 + 3 < t) p3 += a4.w * x[s2 + 3];
+      for (int r = 0; r < 4; ++r) {
+        const int t = 16 * i + 4 * g + r;
+        x[j][i][r] = is_w ? bs[t] * expf(gs[t]) * ks[t][col] : t < n ? bs[t] * x[j][i][r] : 0.f;
       }
-      x[t] -= (p0 + p1) + (p2 + p3);
-    }
-    float *dst = (is_w ? a.wm : a.u) + ch * C * DL + col;
+  }
+  __syncthreads();
 #pragma unroll
-    for (int t = 0; t < C; ++t) dst[t * DL] = x[t];
+  for (int i = 0; i < 4; ++i) {
+    f32x4 acc[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[j] = f32x4{x[j][i][0], x[j][i][1], x[j][i][2], x[j][i][3]};
+#pragma unroll
+    for (int i2 = 0; i2 < i; ++i2) {
+      const float4 m = *(const float4 *)&as[16 * i + r16][16 * i2 + 4 * g];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = mfma4(m.x, x[j][i2][0], acc[j]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = mfma4(m.y, x[j][i2][1], acc[j]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = mfma4(m.z, x[j][i2][2], acc[j]);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = mfma4(m.w, x[j][i2][3], acc[j]);
+    }
+    const float4 d = *(const float4 *)&dinv[i][r16][4 * g];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+      f32x4 y = {0.f, 0.f, 0.f, 0.f};
+      y = mfma4(d.x, acc[j][0], y);
+      y = mfma4(d.y, acc[j][1], y);
+      y = mfma4(d.z, acc[j][2], y);
+      y = mfma4(d.w, acc[j][3], y);
+      const bool is_w = wave + 8 * j >= CT;
+      float *dst = (is_w ? a.wm : a.u) + ch * C * DL + 16 * (wave + 8 * j - (is_w ? CT : 0)) + r16;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        x[j][i][r] = y[r];
+        dst[(16 * i + 4 * g + r) * DL] = y[r];
+      }
+    }
   }
   if (tid < C) a.gam[ch * C + tid] = gs[tid];
 }
 
 // The chunks of one (sequence, head) in order for 16 columns of the state
-// (grid B * Hl * DL / 16, 256 threads). Wave w owns rows 16 w .. 16 w + 15 of
-// the chunk for Delta and O, and state rows 16 it .. + 15 for it = w,
-// w + 4, .. (DL / 64 tiles per wave) for the update. The state and Delta pass
-// between waves through LDS.
+// (grid B * Hl * DL / 16, 512 threads; a head's workgroups B * Hl apart, on
+// one XCD's L2 where that is a multiple of 8). Waves 0 .. 3 walk the state:
+// wave w owns rows 16 w .. + 15 of Delta and state rows 16 it .. + 15 for it =
+// w, w + 4, .. (kept in its registers). Waves 4 .. 7 form the output rows
+// 16 (w - 4) .. + 15 beside them. The state and Delta pass between waves
+// through LDS, columns major (16-byte reads and writes), two barriers a chunk.
+// The serial chain bounds it (64 MFMAs and the two exchanges per 64 positions;
+// the matrix cores are busy 37% of it). At 500 positions, 16 heads of 128: 38.7
+// -> 33 us against four waves doing both parts with three barriers and 4-byte
+// exchanges.
 template <int DL>
 __device__ void delta_scan(const Q35ChunkArgs &a) {
   constexpr int C = 64, KQ = DL / 4, GROUPS = DL / 16, IT = DL / 64;
-  __shared__ float ss[DL][17], ds[C][17];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int r16 = lane & 15, g = lane >> 4;
-  const int bh = blockIdx.x / GROUPS, grp = blockIdx.x - bh * GROUPS;
+  __shared__ __attribute__((aligned(16))) float st[16][DL + 4], ds[16][C + 4];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4, w = wave & 3;
+  const int nbh = gridDim.x / GROUPS, grp = blockIdx.x / nbh, bh = blockIdx.x - grp * nbh;
   const int b = bh / a.Hl, h = bh - b * a.Hl;
   const int c0 = grp * 16;
   const int64_t W = (int64_t)a.Hl * DL;
-  for (int e = tid; e < DL * 17; e += 256) (&ss[0][0])[e] = 0.f;
-  // Operands of one chunk, each loaded a chunk ahead, right after the current
-  // chunk has consumed the registers it goes to:
-  //   wreg / qreg  W and Qg rows of this wave's tile (lane k index KQ (l / 16) + kk)
-  //   preg         P row (lane k index 16 (l / 16) + kk), ureg  U in the output layout
-  //   kreg         KdT rows 16 it + l % 16, columns s = 16 (l / 16) + kk
-  float wreg[KQ], qreg[KQ], preg[16], ureg[4], kreg[IT][16], gend;
-  auto load_wq = [&](int c) {
-    const int64_t ch = (int64_t)bh * a.NC + c;
-    const int t = 16 * wave + r16;
-    const float *wr = a.wm + (ch * C + t) * DL + KQ * g;
-    const float *qr = a.qg + (ch * C + t) * DL + KQ * g;
+  for (int e = tid; e < 16 * (DL + 4); e += 512) (&st[0][0])[e] = 0.f;
+  // (the two roles take their barriers in separate branches, uniform per wave)
+  auto sync = [] { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+  // Operands of one chunk, in two register sets, each loaded two chunks ahead
+  // right after its chunk has consumed it: rows of W / Qg, P and KdT (row
+  // l % 16 of the tile), and U in the output layout. The k index of lane l at
+  // step 4 q + e is 16 q + 4 (l / 16) + e, so four lanes read 64 bytes of a row
+  // together (each lane a piece of its own line, 64 lines an instruction, held
+  // the loop to the L1's line rate: 36 us). (The last chunks re-read the last:
+  // every step issues the same loads, so their waits stay counted.)
+  auto load_row = [&](const float *src, auto &dst) {
+    constexpr int N = sizeof(dst) / sizeof(float);
 #pragma unroll
-    for (int kk = 0; kk < KQ; kk += 4) {
-      const float4 w4 = *(const float4 *)(wr + kk);
-      const float4 q4 = *(const float4 *)(qr + kk);
-      wreg[kk] = w4.x, wreg[kk + 1] = w4.y, wreg[kk + 2] = w4.z, wreg[kk + 3] = w4.w;
-      qreg[kk] = q4.x, qreg[kk + 1] = q4.y, qreg[kk + 2] = q4.z, qreg[kk + 3] = q4.w;
+    for (int kk = 0; kk < N; kk += 4) {
+      const float4 v = *(const float4 *)(src + 4 * kk);
+      dst[kk] = v.x, dst[kk + 1] = v.y, dst[kk + 2] = v.z, dst[kk + 3] = v.w;
     }
   };
-  auto load_pu = [&](int c) {
-    const int64_t ch = (int64_t)bh * a.NC + c;
-    const float *pr = a.pm + (ch * C + 16 * wave + r16) * C + 16 * g;
+  // rows (this lane's operand row) times S0, 16 x 16
+  auto times_state = [&](const float *row) {
+    f32x4 p[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    float4 sv[KQ / 4];
 #pragma unroll
-    for (int kk = 0; kk < 16; kk += 4) {
-      const float4 p4 = *(const float4 *)(pr + kk);
-      preg[kk] = p4.x, preg[kk + 1] = p4.y, preg[kk + 2] = p4.z, preg[kk + 3] = p4.w;
+    for (int q = 0; q < KQ / 4; ++q) sv[q] = *(const float4 *)&st[r16][16 * q + 4 * g];
+    __builtin_amdgcn_sched_barrier(0);  // (all reads out before the first wait)
+#pragma unroll
+    for (int q = 0; q < KQ / 4; ++q) {
+      p[0] = mfma4(row[4 * q], sv[q].x, p[0]);
+      p[1] = mfma4(row[4 * q + 1], sv[q].y, p[1]);
+      p[0] = mfma4(row[4 * q + 2], sv[q].z, p[0]);
+      p[1] = mfma4(row[4 * q + 3], sv[q].w, p[1]);
     }
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ureg[r] = a.u[(ch * C + 16 * wave + 4 * g + r) * DL + c0 + r16];
+    return p[0] + p[1];
   };
-  auto load_k = [&](int c) {
-    const int64_t ch = (int64_t)bh * a.NC + c;
+  auto read_delta = [&](float *dv) {
 #pragma unroll
-    for (int q2 = 0; q2 < IT; ++q2) {
-      const float *kr = a.kdt + (ch * DL + 16 * (wave + 4 * q2) + r16) * C + 16 * g;
-#pragma unroll
-      for (int kk = 0; kk < 16; kk += 4) {
-        const float4 k4 = *(const float4 *)(kr + kk);
-        kreg[q2][kk] = k4.x, kreg[q2][kk + 1] = k4.y, kreg[q2][kk + 2] = k4.z, kreg[q2][kk + 3] = k4.w;
-      }
+    for (int q = 0; q < 4; ++q) {
+      const float4 v = *(const float4 *)&ds[r16][16 * q + 4 * g];
+      dv[4 * q] = v.x, dv[4 * q + 1] = v.y, dv[4 * q + 2] = v.z, dv[4 * q + 3] = v.w;
     }
-    gend = a.gam[ch * C + C - 1];
+    __builtin_amdgcn_sched_barrier(0);
   };
-  load_wq(0);
-  load_pu(0);
-  load_k(0);
-  __syncthreads();
-  for (int c = 0; c < a.NC; ++c) {
-    const int n = min(C, a.S - c * C);
-    const int64_t row0 = (int64_t)b * a.S + c * C;
-    // the next chunk's operands (the last chunk re-reads its own: every
-    // iteration issues the same loads, so the waits for them stay counted)
-    const int cn = min(c + 1, a.NC - 1);
-    // W S0 and Qg S0 (16 x 16 each); the state fragments read first
-    f32x4 wsa, qsa;
-    {
-      float sv[KQ];
-#pragma unroll
-      for (int kk = 0; kk < KQ; ++kk) sv[kk] = ss[KQ * g + kk][r16];
-      f32x4 w2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, q2v[2] = {w2[0], w2[0]};
-#pragma unroll
-      for (int kk = 0; kk < KQ; ++kk) {
-        w2[kk & 1] = mfma4(wreg[kk], sv[kk], w2[kk & 1]);
-        q2v[kk & 1] = mfma4(qreg[kk], sv[kk], q2v[kk & 1]);
-      }
-      wsa = w2[0] + w2[1];
-      qsa = q2v[0] + q2v[1];
-    }
-    load_wq(cn);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ds[16 * wave + 4 * g + r][r16] = ureg[r] - wsa[r];
-    __syncthreads();  // Delta in LDS; every read of S0 for W S0 / Qg S0 done
-    // O = Qg S0 + P Delta (the Delta fragments, read once, also feed the update)
-    float dv[16];
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) dv[kk] = ds[16 * g + kk][r16];
-    f32x4 o = qsa, o2 = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kk = 0; kk < 16; kk += 2) {
-      o = mfma4(preg[kk], dv[kk], o);
-      o2 = mfma4(preg[kk + 1], dv[kk + 1], o2);
-    }
-    o += o2;
-    load_pu(cn);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int t = 16 * wave + 4 * g + r;
-      if (t < n) a.out[(row0 + t) * W + (int64_t)h * DL + c0 + r16] = o[r];
-    }
-    // S_end = Gamma_end S0 + KdT Delta
+  const int64_t ch0 = (int64_t)bh * a.NC;
+  if (wave < 4) {
+    float wreg[2][KQ], ureg[2][4], kreg[2][IT][16];
+    // Gamma_end of every chunk, one a lane (at most 64: sequences are up to 4096)
+    const float decay = expf(a.gam[(ch0 + min(lane, a.NC - 1)) * C + C - 1]);
     f32x4 sn[IT];
-    const float eg = expf(gend);
+    auto load_w = [&](int c, int s) { load_row(a.wm + ((ch0 + c) * C + 16 * w + r16) * DL + 4 * g, wreg[s]); };
+    auto load_u = [&](int c, int s) {
 #pragma unroll
-    for (int q2 = 0; q2 < IT; ++q2) {
-      const int it = wave + 4 * q2;
+      for (int r = 0; r < 4; ++r) ureg[s][r] = a.u[((ch0 + c) * C + 16 * w + 4 * g + r) * DL + c0 + r16];
+    };
+    auto load_k = [&](int c, int s) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sn[q2][r] = eg * ss[16 * it + 4 * g + r][r16];
-      f32x4 s2v = {0.f, 0.f, 0.f, 0.f};
+      for (int q2 = 0; q2 < IT; ++q2)
+        load_row(a.kdt + ((ch0 + c) * DL + 16 * (w + 4 * q2) + r16) * C + 4 * g, kreg[s][q2]);
+    };
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int c = min(s, a.NC - 1);
+      load_w(c, s);
+      load_u(c, s);
+      load_k(c, s);
+    }
+#pragma unroll
+    for (int q2 = 0; q2 < IT; ++q2) sn[q2] = f32x4{0.f, 0.f, 0.f, 0.f};
+    sync();
+    auto step = [&](int c, int s) {
+      const int cn = min(c + 2, a.NC - 1);
+      const f32x4 wsa = times_state(wreg[s]);
+      *(f32x4 *)&ds[r16][16 * w + 4 * g] = f32x4{ureg[s][0], ureg[s][1], ureg[s][2], ureg[s][3]} - wsa;
+      load_w(cn, s);
+      load_u(cn, s);
+      sync();  // Delta in LDS; every read of S0 done
+      float dv[16];
+      read_delta(dv);
+      // S_end = Gamma_end S0 + KdT Delta
+      const float eg = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, decay), c));
+      f32x4 s2v[IT];
+#pragma unroll
+      for (int q2 = 0; q2 < IT; ++q2) sn[q2] *= eg, s2v[q2] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < 16; kk += 2)
+#pragma unroll
+        for (int q2 = 0; q2 < IT; ++q2) {
+          sn[q2] = mfma4(kreg[s][q2][kk], dv[kk], sn[q2]);
+          s2v[q2] = mfma4(kreg[s][q2][kk + 1], dv[kk + 1], s2v[q2]);
+        }
+#pragma unroll
+      for (int q2 = 0; q2 < IT; ++q2) {
+        sn[q2] += s2v[q2];
+        *(f32x4 *)&st[r16][16 * (w + 4 * q2) + 4 * g] = sn[q2];
+      }
+      load_k(cn, s);
+      sync();  // the new state in LDS; Delta free
+    };
+    for (int c = 0; c < a.NC; c += 2) {
+      step(c, 0);
+      if (c + 1 >= a.NC) break;
+      step(c + 1, 1);
+    }
+  } else {
+    float qreg[2][KQ], preg[2][16];
+    auto load_q = [&](int c, int s) { load_row(a.qg + ((ch0 + c) * C + 16 * w + r16) * DL + 4 * g, qreg[s]); };
+    auto load_p = [&](int c, int s) { load_row(a.pm + ((ch0 + c) * C + 16 * w + r16) * C + 4 * g, preg[s]); };
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int c = min(s, a.NC - 1);
+      load_q(c, s);
+      load_p(c, s);
+    }
+    sync();
+    auto step = [&](int c, int s) {
+      const int n = min(C, a.S - c * C), cn = min(c + 2, a.NC - 1);
+      const int64_t row0 = (int64_t)b * a.S + c * C;
+      // O = Qg S0 + P Delta
+      f32x4 o = times_state(qreg[s]), o2 = {0.f, 0.f, 0.f, 0.f};
+      load_q(cn, s);
+      sync();
+      float dv[16];
+      read_delta(dv);
 #pragma unroll
       for (int kk = 0; kk < 16; kk += 2) {
-        sn[q2] = mfma4(kreg[q2][kk], dv[kk], sn[q2]);
-        s2v = mfma4(kreg[q2][kk + 1], dv[kk + 1], s2v);
+        o = mfma4(preg[s][kk], dv[kk], o);
+        o2 = mfma4(preg[s][kk + 1], dv[kk + 1], o2);
       }
-      sn[q2] += s2v;
-    }
-    load_k(cn);
-    __syncthreads();  // every read of S0 done
+      o += o2;
+      load_p(cn, s);
+      sync();
 #pragma unroll
-    for (int q2 = 0; q2 < IT; ++q2) {
-      const int it = wave + 4 * q2;
-#pragma unroll
-      for (int r = 0; r < 4; ++r) ss[16 * it + 4 * g + r][r16] = sn[q2][r];
+      for (int r = 0; r < 4; ++r) {
+        const int t = 16 * w + 4 * g + r;
+        if (t < n) a.out[(row0 + t) * W + (int64_t)h * DL + c0 + r16] = o[r];
+      }
+    };
+    for (int c = 0; c < a.NC; c += 2) {
+      step(c, 0);
+      if (c + 1 >= a.NC) break;
+      step(c + 1, 1);
     }
-    __syncthreads();  // the new state in LDS; Delta free
   }
 }
 
 #define RXW8_Q35_CHUNK(DL)                                                         \
-  extern "C" __global__ void __launch_bounds__(256) rxw8_q35_delta_chunk_d##DL(Q35ChunkArgs a) { \
+  extern "C" __global__ void __launch_bounds__(512) rxw8_q35_delta_chunk_d##DL(Q35ChunkArgs a) { \
     delta_chunk<DL>(a);                                                            \
   }                                                                                \
-  extern "C" __global__ void __launch_bounds__(256) rxw8_q35_delta_scan_d##DL(Q35ChunkArgs a) { \
+  extern "C" __global__ void __launch_bounds__(512) rxw8_q35_delta_scan_d##DL(Q35ChunkArgs a) { \
     delta_scan<DL>(a);                                                             \
   }
 RXW8_Q35_CHUNK(64)

@@ -153,6 +153,22 @@ def test_chunked_delta_rule(rt, monkeypatch, name, b, s):
     assert e_pair <= 1e-4
 
 
+def test_chunked_delta_rule_longest(rt, monkeypatch):
+    """The longest sequence but a few: 64 chunks, one decay per lane of the
+    walk. Against the sequential recurrence (itself held to the oracle above),
+    to the same 1e-4 between the two orders of summation."""
+    cfg = dict(CONFIGS["mid"], layers=[q35.LINEAR], max_batch=1, max_seq=4096)
+    p = q35.random_params(cfg, seed=63, std=0.05)
+    ids = np.random.default_rng(64).integers(0, cfg["vocab"], (1, 4090))
+    monkeypatch.setenv("RXW8_Q35_SHORT", "0")
+    monkeypatch.setenv("RXW8_Q35_CHUNKED", "1")
+    chunked = run(rt, build(rt, cfg, p), ids)
+    monkeypatch.setenv("RXW8_Q35_CHUNKED", "0")
+    seq = run(rt, build(rt, cfg, p), ids)
+    assert np.isfinite(chunked).all()
+    assert rel_err(chunked, seq) <= 1e-4
+
+
 @pytest.mark.parametrize("name,b,s", [("mid_long", 2, 150), ("wide_full", 1, 160)])
 def test_f32_gemm_split_k_residuals(rt, monkeypatch, name, b, s):
     """Every F32 projection that fits the GEMM tiles forced onto them
