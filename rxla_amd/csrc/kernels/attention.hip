@@ -1238,12 +1238,11 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
       lds_dma16_asm(a.vc + kv_base, (uint32_t)key * (2 * D) + vx, dst + 4096 * HW * n);
     }
   };
-  // the first copies go out before anything else (q's loads overlap them)
-  // K blocks 0 .. NB - 1, V blocks 0 .. NB - 2
-  for (int j = 0; j < NB; ++j) {
-    if (j < nblk) dma_k(j);
-    if (j < nblk && j < NB - 1) dma_v(j);
-  }
+  // what the first block needs goes out before anything else (q's loads
+  // overlap it), the rest of the rings once q is here
+  dma_k(0);
+  dma_v(0);
+  if (nblk > 1) dma_k(1);
 
   // p = exp(scale s - m) = exp2(c s - m'), c = scale * log2(e) > 0. (Below
   // 1e-30 every visible key weighs the same either way; a masked key's c (-inf)
@@ -1284,6 +1283,18 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
     for (int r = 0; r < R; ++r)
 #pragma unroll
       for (int t = 0; t < 4; ++t) qhi[r][t] = *(const u32x4 *)((const uint16_t *)a.q + q_row[r] + 32 * t);
+  }
+
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) asm volatile("" : "+v"(qhi[r][t]));  // (waited for here)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  // K blocks 2 .. NB - 1 and V blocks 1 .. NB - 2, in the order of the steps below
+#pragma unroll
+  for (int j = 2; j < NB; ++j) {
+    if (j < nblk) dma_k(j);
+    if (j - 1 < nblk) dma_v(j - 1);
   }
 
   f32x4 o[R][8];
@@ -1474,7 +1485,7 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
   };
   static_assert(HW == 1 || (NB == 4 && 8 / HW * (NB - 2) == 8), "the wait's count");
 
-  sync(true, nblk);
+  sync(false, 0);  // (every wave's first copies are in: waited for with q)
   if (ph) sync(false, 0);  // the second head's waves run half a step later
   auto to_vector = [&](int blk) {
     if (HW == 2) sync(ph, blk);
