@@ -1160,8 +1160,10 @@ __device__ void delta_scan(const Q35ChunkArgs &a) {
   const int64_t ch0 = (int64_t)bh * a.NC;
   if (wave < 4) {
     float wreg[2][KQ], ureg[2][4], kreg[2][IT][16];
-    // Gamma_end of every chunk, one a lane (at most 64: sequences are up to 4096)
-    const float decay = expf(a.gam[(ch0 + min(lane, a.NC - 1)) * C + C - 1]);
+    // Gamma_end of 64 chunks at a time, one a lane (read again at every 64th chunk)
+    float decay;
+    auto load_decay = [&](int c) { decay = expf(a.gam[(ch0 + min(c + lane, a.NC - 1)) * C + C - 1]); };
+    load_decay(0);
     f32x4 sn[IT];
     auto load_w = [&](int c, int s) { load_row(a.wm + ((ch0 + c) * C + 16 * w + r16) * DL + 4 * g, wreg[s]); };
     auto load_u = [&](int c, int s) {
@@ -1193,7 +1195,7 @@ __device__ void delta_scan(const Q35ChunkArgs &a) {
       float dv[16];
       read_delta(dv);
       // S_end = Gamma_end S0 + KdT Delta
-      const float eg = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, decay), c));
+      const float eg = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, decay), c & 63));
       f32x4 s2v[IT];
 #pragma unroll
       for (int q2 = 0; q2 < IT; ++q2) sn[q2] *= eg, s2v[q2] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1213,6 +1215,7 @@ __device__ void delta_scan(const Q35ChunkArgs &a) {
       sync();  // the new state in LDS; Delta free
     };
     for (int c = 0; c < a.NC; c += 2) {
+      if (c > 0 && (c & 63) == 0) load_decay(c);
       step(c, 0);
       if (c + 1 >= a.NC) break;
       step(c + 1, 1);

@@ -153,20 +153,29 @@ def test_chunked_delta_rule(rt, monkeypatch, name, b, s):
     assert e_pair <= 1e-4
 
 
-def test_chunked_delta_rule_longest(rt, monkeypatch):
-    """The longest sequence but a few: 64 chunks, one decay per lane of the
-    walk. Against the sequential recurrence (itself held to the oracle above),
-    to the same 1e-4 between the two orders of summation."""
-    cfg = dict(CONFIGS["mid"], layers=[q35.LINEAR], max_batch=1, max_seq=4096)
+@pytest.mark.parametrize("s", [4090, 4160, 4200, 5000, 8200])
+def test_chunked_delta_rule_many_chunks(rt, monkeypatch, s):
+    """More chunks than a wave has lanes (the walk holds 64 chunks' decays at
+    a time): 64 chunks, 65, 66 (the first one after chunk 64's decay), 79 and
+    129. Against the sequential recurrence (itself held to the oracle above), to the same 1e-4
+    between the two orders of summation, over the positions of each run of 64
+    chunks by themselves. The heads forget slowly (a chunk leaves 0.7 down to
+    2e-3 of the state it began with, by its own tokens), so that a chunk's
+    decay shows in the outputs after it."""
+    cfg = dict(CONFIGS["mid"], layers=[q35.LINEAR], max_batch=1, max_seq=s, max_positions=16384)
     p = q35.random_params(cfg, seed=63, std=0.05)
-    ids = np.random.default_rng(64).integers(0, cfg["vocab"], (1, 4090))
+    for path in p:
+        if path.endswith("A_log"):
+            p[path] = np.linspace(-5, -2, p[path].size, dtype=np.float32)
+    ids = np.random.default_rng(64).integers(0, cfg["vocab"], (1, s))
     monkeypatch.setenv("RXW8_Q35_SHORT", "0")
     monkeypatch.setenv("RXW8_Q35_CHUNKED", "1")
     chunked = run(rt, build(rt, cfg, p), ids)
     monkeypatch.setenv("RXW8_Q35_CHUNKED", "0")
     seq = run(rt, build(rt, cfg, p), ids)
     assert np.isfinite(chunked).all()
-    assert rel_err(chunked, seq) <= 1e-4
+    for lo in range(0, s, 4096):
+        assert rel_err(chunked[:, lo:lo + 4096], seq[:, lo:lo + 4096]) <= 1e-4
 
 
 @pytest.mark.parametrize("name,b,s", [("mid_long", 2, 150), ("wide_full", 1, 160)])
