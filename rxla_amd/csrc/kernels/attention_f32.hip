@@ -522,13 +522,12 @@ __device__ void gqa_tile(const GqaTileArgs &a) {
         p[c] = 16 * t + 4 * j + c < row.vis ? s : kNegInf;
       }
       softmax_step<D>(st, p);
-      // a key that some row of the wave must not see (causal starts) may hold
-      // anything: a product 0 x NaN would reach that row, so such a tile's
-      // products are formed per row and key
+      // a key that some row of the wave must not see (one past a causal row's,
+      // or the last key again in the rows a tile has past it) may hold
+      // anything: a product 0 x NaN or 0 x inf would reach that row, so such a
+      // tile's products are formed per row and key
       bool plain = true;
-      if (a.starts && 16 * t + 16 > vis_min) {
-        plain = below<BF, TILEB>(vt, lane, kInfBits);
-      }
+      if (16 * t + 16 > vis_min) plain = below<BF, TILEB>(vt, lane, kInfBits);
       if (plain) {
         if constexpr (!PRE) read_v(0), read_v(1);
         if constexpr (D == 256) read_v(2), read_v(3);
@@ -778,7 +777,7 @@ __device__ void gqa_quad(const GqaTileArgs &a) {
       l[s] += p[s];
     }
     bool plain = true;
-    if (a.starts && 16 * t + 16 > vis_min) {  // keys that some row must not see (see gqa_tile)
+    if (16 * t + 16 > vis_min) {  // keys that some row must not see (see gqa_tile)
       // (on the raw bits: sharing the widened values with the products would
       // keep them all in registers)
       uint32_t hi = 0, lo = 0;

@@ -155,6 +155,58 @@ def test_not_a_number_and_infinities_as_the_scalar_kernel(rt, monkeypatch, sq, h
     assert np.max(np.abs(got[ok] - want[ok])) <= 2e-5
 
 
+def same_non_numbers(got, want):
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
+    np.testing.assert_array_equal(np.isinf(got), np.isinf(want))
+    np.testing.assert_array_equal(got[np.isinf(got)], want[np.isinf(want)])
+    ok = np.isfinite(want)
+    assert np.max(np.abs(got[ok] - want[ok])) <= 2e-5
+
+
+@pytest.mark.parametrize("sk", [1, 16, 70])
+@pytest.mark.parametrize("d,sq,hq", [(64, 1, 4), (128, 4, 4), (256, 40, 2), (128, 40, 4)])
+def test_infinite_value_of_the_last_key(rt, monkeypatch, d, sq, hq, sk):
+    """The last key's row stands in for the rows that a 16-key tile has past
+    it, with weight 0: an infinity there reaches the outputs as itself, as in
+    the scalar kernel, and not as 0 x inf."""
+    r = rx()
+    rng = np.random.default_rng(sk + d)
+    q = rng.standard_normal((2, hq, sq, d)).astype(np.float32)
+    k = rng.standard_normal((2, 2, sk, d)).astype(np.float32)
+    v = rng.standard_normal((2, 2, sk, d)).astype(np.float32)
+    v[0, 1, sk - 1, :3], v[1, 0, sk - 1, d - 2:] = np.inf, -np.inf
+    bufs = [rt.buffer(x) for x in (q, k, v, rng.standard_normal((2, 1, sq, sk)).astype(np.float32))]
+    for rg in ("4", "2"):
+        monkeypatch.setenv("RXW8_ATTN_F32_RG", rg)
+        for mask in (bufs[3], None):
+            got = r.gqa_attention(rt, *bufs[:3], mask).to_numpy()
+            with monkeypatch.context() as m:
+                m.setenv("RXW8_FORCE_GENERIC", "1")
+                want = r.gqa_attention(rt, *bufs[:3], mask).to_numpy()
+            assert np.isinf(want).any() and not np.isnan(want).any()
+            same_non_numbers(got, want)
+
+
+@pytest.mark.parametrize("d,cache", [(64, "bf16"), (256, "bf16"), (128, "f32")])
+@pytest.mark.parametrize("hq", [2, 16])
+def test_infinite_value_of_the_last_key_in_decode(rt, monkeypatch, d, cache, hq):
+    r = rx()
+    rng = np.random.default_rng(d + hq)
+    lens = np.array([1, 16, 33, 70], np.int32)
+    q = rng.standard_normal((4, hq, d)).astype(np.float32)
+    k = oracle.round_bf16(rng.standard_normal((4, 1, 80, d)).astype(np.float32))
+    v = oracle.round_bf16(rng.standard_normal((4, 1, 80, d)).astype(np.float32))
+    for i in range(4):
+        v[i, 0, lens[i] - 1, :3] = np.inf
+    bits = (lambda x: rt.buffer(oracle.bf16_bits(x), r.DType.BF16)) if cache == "bf16" else rt.buffer
+    bufs = (rt.buffer(q), bits(k), bits(v), rt.buffer(lens))
+    got = r.grouped_query_attention(rt, *bufs).to_numpy()
+    monkeypatch.setenv("RXW8_FORCE_GENERIC", "1")
+    want = r.grouped_query_attention(rt, *bufs).to_numpy()
+    assert np.isposinf(want[:, :, :3]).all() and np.isfinite(want[:, :, 3:]).all()
+    same_non_numbers(got, want)
+
+
 def test_decode_in_a_capture_uses_no_workspace(rt):
     """A captured decode call runs without the split workspace, which a later
     call may free: replays agree with the eager result, also after one."""
