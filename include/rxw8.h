@@ -243,10 +243,11 @@ int rxw8_causal_attention_mask(rxw8_runtime *rt, rxw8_buffer *query_positions,
  * (RXW8_NOALLOC_PARTIAL_BYTES + RXW8_NOALLOC_COUNTER_BYTES); a call whose plan
  * needs more fails with RXW8_RESOURCE_EXHAUSTED before any launch. The split
  * plans of the D = 128 kernel (Hq/Hkv in {1, 2, 4, 8}) use at most 4 x CUs
- * partial slots of Hq/Hkv x 130 floats -- 4.1 MiB on 256 CUs -- and the
- * other kernels' plans never exceed the array, so on MI355X that happens only
- * for a counter need (rows x kv heads) above 16384 of the D = 128 kernel.
- * Every call on one GPU shares that array: calls that overlap on one GPU
+ * partial slots of Hq/Hkv x 130 floats -- 4.1 MiB on 256 CUs -- and those of
+ * the f32 kernels (f32 caches, D = 64 and 256) are cut to what the array
+ * holds, so on MI355X that happens only for a counter need (rows x kv heads)
+ * above 16384 of the D = 128 kernel. Every call on one GPU, over whichever
+ * cache and head width, shares that array: calls that overlap on one GPU
  * (other streams, runtimes or threads) race and must be serialised by the
  * caller. The device must have had a runtime created on it (set-up). */
 #define RXW8_NOALLOC_PARTIAL_BYTES ((size_t)16 << 20)

@@ -68,6 +68,10 @@ struct AttnRope {
   float eps;                     // the new token of row r sits at lens[r] - 1
 };
 
+// Counters, then partials: what the no-allocation entry's array holds, so that
+// both entries run one plan.
+constexpr size_t kF32AttnBlock = RXW8_NOALLOC_COUNTER_BYTES + RXW8_NOALLOC_PARTIAL_BYTES;
+
 struct Runtime;
 
 struct Buffer {
@@ -115,6 +119,10 @@ struct Runtime {
   Workspace xcast;     // bf16 copy of f32 activations ahead of the GEMM
   Workspace wdeq;      // bf16 dequantised weights ahead of the large-M GEMM
   Workspace attn_counters;  // i32 split arrival counters of decode attention (zeroed once)
+  // Split counters and partials of the f32 attention kernels, fixed blocks of
+  // kF32AttnBlock bytes (kernels/attention_f32.hip): of calls that run, and of
+  // calls that a capture records
+  char *f32_attn[2] = {nullptr, nullptr};
 
   hipFunction_t fn(const char *name);
 };

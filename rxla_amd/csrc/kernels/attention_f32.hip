@@ -58,6 +58,16 @@ struct GqaTileArgs {
   int q_bf16, out_bf16;
 };
 
+// Split partials and counters of a runtime's calls, one block for calls that
+// run and one for calls that a stream capture records (16 MiB and 64 KiB each,
+// as the no-allocation entry's array). This code object is loaded once per
+// runtime, so each runtime has its own, and a captured pointer is good until
+// the runtime ends: no later call moves the block, and none that runs beside a
+// replay uses it. runtime_create takes the address and clears the counters.
+extern "C" {
+__attribute__((used)) __device__ __align__(256) unsigned char rxw8_f32_attention_blocks[2][(64 << 10) + (16 << 20)];
+}
+
 namespace {
 
 constexpr float kNegInf = -__builtin_huge_valf();

@@ -1220,8 +1220,7 @@ int bf16_linear_launch(Runtime *rt, const void *x, int x_f32, const uint16_t *w,
   return run_generic_linear(rt, x, x_f32, w, 1, nullptr, y, y_f32, M, N, K, K, 1);
 }
 
-// Split partials and counters of one f32 attention launch at most: what the
-// no-allocation entry's fixed array holds, so that both entries run one plan.
+// Split partials and counters of one f32 attention launch at most (kF32AttnBlock)
 constexpr size_t kF32PartialMax = RXW8_NOALLOC_PARTIAL_BYTES;
 constexpr int64_t kF32UnitsMax = RXW8_NOALLOC_COUNTER_BYTES / sizeof(int);
 
@@ -1284,26 +1283,18 @@ static int attention_f32_launch(Runtime *rt, GqaTileArgs a, int64_t D, int64_t D
   if (forced > 0) S = std::min<int64_t>(forced, 32);
   S = std::min<int64_t>(S, 32);
   const size_t per_split = (size_t)(units * rows) * (size_t)(4 + D) * sizeof(float);
-  // One workgroup per unit where the split workspace must not be used: in a
-  // stream capture (the graph would keep a pointer that a later, larger call
-  // frees), and for the decoder plan (slots), whose captured step runs the
-  // same plan as its eager one.
-  if (units > kF32UnitsMax || a.slots || (!ext && stream_capturing(rt))) S = 1;
+  // One plan for the running, the captured and the no-allocation call, whose
+  // results are the same bits: all three blocks hold kF32PartialMax and
+  // kF32UnitsMax. (The decoder plan, slots, keeps one workgroup per unit.)
+  if (units > kF32UnitsMax || a.slots) S = 1;
   if (S > 1) S = std::max<int64_t>(1, std::min<int64_t>(S, (int64_t)(kF32PartialMax / per_split)));
   if (units * S >= ((int64_t)1 << 31)) return RXW8_UNIMPLEMENTED;
   if (S > 1) {
-    const size_t need_p = per_split * (size_t)S, need_c = (size_t)units * sizeof(int);
-    if (ext) {
-      a.part = ext->partials;
-      a.counters = ext->counters;
-      if (need_p > ext->partial_bytes || need_c > ext->counter_bytes) S = 1;
-    } else if (ensure_workspace(rt, rt->scratch, need_p, false) ||
-               ensure_workspace(rt, rt->attn_counters, need_c, true)) {
-      S = 1;  // no memory for it: one workgroup per unit needs none
-    } else {
-      a.part = (float *)rt->scratch.ptr;
-      a.counters = (int *)rt->attn_counters.ptr;
-    }
+    char *block = ext ? nullptr : rt->f32_attn[stream_capturing(rt) ? 1 : 0];
+    a.counters = ext ? ext->counters : (int *)block;
+    a.part = ext ? ext->partials : (float *)(block + RXW8_NOALLOC_COUNTER_BYTES);
+    if (ext && (per_split * (size_t)S > ext->partial_bytes || (size_t)units * sizeof(int) > ext->counter_bytes))
+      return fail(RXW8_RESOURCE_EXHAUSTED, "decode attention: the workspace is smaller than the split plan's");
   }
   a.nsplit = (int)S;
   char kname[40];

@@ -269,6 +269,23 @@ int rxw8_status_is_retryable(int status) {
 
 int rxw8_abi_version(void) { return RXW8_ABI_VERSION; }
 
+// The f32 attention blocks of the loaded code object, their counters cleared
+// and waited for on the runtime's own new stream.
+static int f32_attention_setup(Runtime *rt) {
+  hipDeviceptr_t p = nullptr;
+  size_t bytes = 0;
+  RXW8_HIP(hipModuleGetGlobal(&p, &bytes, rt->modules[(size_t)module_of("rxw8_gqa_tile_")],
+                              "rxw8_f32_attention_blocks"));
+  if (bytes != 2 * kF32AttnBlock)
+    return fail(RXW8_INTERNAL, "the f32 attention blocks hold %zu bytes, not %zu", bytes, 2 * kF32AttnBlock);
+  for (int i = 0; i < 2; ++i) {
+    rt->f32_attn[i] = (char *)p + i * kF32AttnBlock;
+    RXW8_HIP(hipMemsetAsync(rt->f32_attn[i], 0, RXW8_NOALLOC_COUNTER_BYTES, rt->own_stream));
+  }
+  RXW8_HIP(hipStreamSynchronize(rt->own_stream));
+  return RXW8_OK;
+}
+
 int rxw8_runtime_create(int device, rxw8_runtime **out) {
   if (!out) return fail(RXW8_INVALID_ARGUMENT, "out is NULL");
   *out = nullptr;
@@ -327,7 +344,8 @@ int rxw8_runtime_create(int device, rxw8_runtime **out) {
     return rc;
   }
   rt->stream = rt->own_stream;
-  if (int rc = noalloc_device_setup(device, rt->own_stream)) {
+  int rc = f32_attention_setup(rt);
+  if (rc || (rc = noalloc_device_setup(device, rt->own_stream))) {
     (void)hipStreamDestroy(rt->own_stream);
     for (hipModule_t mm : rt->modules) (void)hipModuleUnload(mm);
     delete rt;

@@ -207,34 +207,72 @@ def test_infinite_value_of_the_last_key_in_decode(rt, monkeypatch, d, cache, hq)
     same_non_numbers(got, want)
 
 
-def test_decode_in_a_capture_uses_no_workspace(rt):
-    """A captured decode call runs without the split workspace, which a later
-    call may free: replays agree with the eager result, also after one."""
+def captured(own, call):
+    """The graph of call() on a stream of its own that stays the runtime's
+    (call has run eagerly there first)."""
+    import torch
+    stream = torch.cuda.Stream()
+    own.synchronize()
+    own.set_stream(stream.cuda_stream)
+    call()
+    own.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=stream, capture_error_mode="thread_local"):
+        call()
+    return g, stream
+
+
+@pytest.mark.parametrize("kind", ["decode", "decode-noalloc", "decode-d128", "masked", "prefill"])
+def test_captured_calls_replay_beside_larger_ones(rt, kind):
+    """A captured call gives the bits of the eager one (and the no-allocation
+    decode call those of the other), at every replay, also with larger calls
+    between and beside the replays: a captured call's split workspace is
+    neither moved nor used by them. decode-d128 is the bf16 flash kernel, whose
+    workspace the f32 kernels leave alone."""
     import torch
     r = rx()
     own = r.Runtime(0)
     rng = np.random.default_rng(3)
-    q = rng.standard_normal((2, 8, 256)).astype(np.float32)
-    k = rng.standard_normal((2, 2, 700, 256)).astype(np.float32)
-    v = rng.standard_normal((2, 2, 700, 256)).astype(np.float32)
-    lens = np.array([700, 333], np.int32)
-    bufs = [own.buffer(x) for x in (q, k, v, lens)]
-    out = own.zeros(q.shape, r.DType.F32)
-    stream = torch.cuda.Stream()
+    d, dt = (128, r.DType.BF16) if kind == "decode-d128" else (256, r.DType.F32)
+    f = lambda *shape: rng.standard_normal(shape).astype(np.float32)  # noqa: E731
+    buf = lambda x: own.buffer(oracle.bf16_bits(x), dt) if dt == r.DType.BF16 else own.buffer(x)  # noqa: E731
+    if kind == "masked":
+        bufs = [own.buffer(x) for x in (f(1, 4, 20, 256), f(1, 2, 600, 256), f(1, 2, 600, 256), f(1, 1, 20, 600))]
+        out = own.zeros((1, 4, 20, 256), r.DType.F32)
+        call = lambda: r.gqa_attention(own, *bufs, out=out)  # noqa: E731
+    elif kind == "prefill":
+        kv = [own.buffer(oracle.bf16_bits(f(1, 2, 700, 64)), r.DType.BF16) for _ in range(2)]
+        bufs = [own.buffer(f(1, 9, 8, 64)), *kv, own.buffer(np.array([600], np.int32))]
+        out = own.zeros((1, 9, 8, 64), r.DType.F32)
+        call = lambda: r.grouped_query_attention_prefill(own, *bufs, out=out)  # noqa: E731
+    else:
+        bufs = [own.buffer(f(2, 8, d)), buf(f(2, 2, 700, d)), buf(f(2, 2, 700, d)),
+                own.buffer(np.array([700, 333], np.int32))]
+        out = own.zeros((2, 8, d), r.DType.F32)
+        fn = r.grouped_query_attention_noalloc if kind == "decode-noalloc" else r.grouped_query_attention
+        call = lambda: fn(own, *bufs, out=out)  # noqa: E731
+    if kind == "decode-noalloc":
+        eager = r.grouped_query_attention(own, *bufs).to_numpy()
+    else:
+        call()
+        eager = out.to_numpy()
+    g, stream = captured(own, call)
+    big = [own.buffer(x) for x in (f(8, 64, 256), f(8, 8, 2048, 256), f(8, 8, 2048, 256))]
+    big_lens, big_out = own.buffer(np.full(8, 2048, np.int32)), own.zeros((8, 64, 256), r.DType.F32)
+    prompt = [own.buffer(x) for x in (f(1, 16, 70, 128), f(1, 2, 4000, 128), f(1, 2, 4000, 128))]
     own.synchronize()
-    own.set_stream(stream.cuda_stream)
-    r.grouped_query_attention(own, *bufs, out=out)
-    own.synchronize()
-    eager = out.to_numpy()
-    g = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, stream=stream, capture_error_mode="thread_local"):
-        r.grouped_query_attention(own, *bufs, out=out)
-    big = [own.buffer(np.zeros(s, np.float32)) for s in ((16, 64, 128), (16, 8, 2048, 128), (16, 8, 2048, 128))]
-    for _ in range(3):
-        out.copy_from(np.full(q.shape, 7.0, np.float32))
-        g.replay()
+    own.set_stream(None)  # eager calls on a stream of their own from here on
+    want = r.grouped_query_attention(own, *big, big_lens).to_numpy()
+    for _ in range(4):
+        out.copy_from(np.full(out.shape, 7.0, np.float32))
         torch.cuda.synchronize()
-        assert rel_err(out.to_numpy(), eager) <= 1e-5
-        r.grouped_query_attention(own, *big, own.buffer(np.full(16, 2048, np.int32)))  # grows the workspace
-        own.synchronize()
-    own.set_stream(None)
+        with torch.cuda.stream(stream):
+            g.replay()
+            g.replay()
+        if kind != "decode-d128":  # beside the replays
+            r.grouped_query_attention(own, *big, big_lens, out=big_out)
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(out.to_numpy(), eager)
+        r.grouped_query_attention(own, *big, big_lens, out=big_out)
+        r.gqa_attention(own, *prompt, None)
+        np.testing.assert_array_equal(big_out.to_numpy(), want)
