@@ -901,7 +901,9 @@ int rxw8_decoder_generate(rxw8_decoder *d, rxw8_buffer *prompt, int64_t b, int64
       d->graph = nullptr;
       d->g_key[0] = -1;
       RXW8_HIP(hipStreamBeginCapture(rt->stream, hipStreamCaptureModeThreadLocal));
+      rt->plan_capture = true;
       rc = step();
+      rt->plan_capture = false;
       hipGraph_t graph = nullptr;
       hipError_t e = hipStreamEndCapture(rt->stream, &graph);
       if (rc) {

@@ -92,10 +92,12 @@ struct Buffer {
   }
 };
 
-// A split-K / scratch workspace owned by the runtime; grown on demand.
+// A split-K / scratch workspace owned by the runtime; grown on demand. `held`:
+// a caller's capture has recorded its address (see ensure_workspace).
 struct Workspace {
   void *ptr = nullptr;
   size_t bytes = 0;
+  bool held = false;
 };
 
 struct Runtime {
@@ -123,6 +125,9 @@ struct Runtime {
   // kF32AttnBlock bytes (kernels/attention_f32.hip): of calls that run, and of
   // calls that a capture records
   char *f32_attn[2] = {nullptr, nullptr};
+
+  std::vector<void *> retired;  // replaced workspace blocks that a caller's graph may hold
+  bool plan_capture = false;    // a plan captures its own step (it replays only while its addresses hold)
 
   hipFunction_t fn(const char *name);
 };
@@ -167,6 +172,10 @@ int noalloc_device_setup(int device, hipStream_t stream);
 // Device-side allocation through the runtime's cache.
 int rt_alloc(Runtime *rt, size_t bytes, void **out);
 void rt_free(Runtime *rt, void *ptr, size_t bytes);
+// At least `bytes` at ws.ptr (cleared once where `zero`). A block that is too
+// small is replaced, which a stream capture cannot do (FAILED_PRECONDITION).
+// Replaying a caller's graph writes to the blocks that its capture recorded:
+// they are kept until the runtime ends.
 int ensure_workspace(Runtime *rt, Workspace &ws, size_t bytes, bool zero);
 // Whether the runtime's stream is being captured into a graph
 bool stream_capturing(const Runtime *rt);

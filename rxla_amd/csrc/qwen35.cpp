@@ -898,7 +898,9 @@ int run_forward(Qwen35 *m, const int32_t *ids, float *logits, int64_t B, int64_t
   if (no_graph || m->g_calls < 2) return enqueue_forward(m, ids, logits, B, S);
   if (!m->gexec) {
     RXW8_HIP(hipStreamBeginCapture(rt->stream, hipStreamCaptureModeThreadLocal));
+    rt->plan_capture = true;
     const int rc = enqueue_forward(m, ids, logits, B, S);
+    rt->plan_capture = false;
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(rt->stream, &graph);
     if (rc) {

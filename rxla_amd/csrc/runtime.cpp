@@ -6,6 +6,7 @@
 // retain their runtime (Buffer/BufferInner :1446,:1523), status codes follow
 // PJRT_Error_Code (vendor/xla/pjrt/c/pjrt_c_api.h:168-186) and
 // PjrtErrorCode::is_retryable (:93-104).
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -163,7 +164,10 @@ bool stream_capturing(const Runtime *rt) {
 }
 
 int ensure_workspace(Runtime *rt, Workspace &ws, size_t bytes, bool zero) {
-  if (ws.bytes >= bytes) return RXW8_OK;
+  if (ws.bytes >= bytes) {
+    if (!ws.held && !rt->plan_capture) ws.held = stream_capturing(rt);
+    return RXW8_OK;
+  }
   // Growing synchronizes the stream and reallocates: not possible inside a
   // stream capture (an XLA command buffer, a caller's graph). Such callers
   // run the call once outside capture first, which sizes the workspace.
@@ -172,14 +176,28 @@ int ensure_workspace(Runtime *rt, Workspace &ws, size_t bytes, bool zero) {
                 "a workspace of %zu bytes (now %zu) must grow while the stream is being captured; "
                 "run the call once outside the capture first",
                 bytes, ws.bytes);
-  if (ws.ptr) {
+  const size_t need = round_size(bytes < (1u << 20) ? (1u << 20) : bytes);
+  size_t want = need;
+  if (ws.held) {
+    // at least doubled, so that the retired blocks together stay below the live one
+    want = std::max(need, round_size(2 * ws.bytes));
+    rt->retired.push_back(ws.ptr);
+    ws = Workspace{};
+  } else if (ws.ptr) {
     RXW8_HIP(hipStreamSynchronize(rt->stream));
     RXW8_HIP(hipFree(ws.ptr));
-    ws.ptr = nullptr;
-    ws.bytes = 0;
+    ws = Workspace{};
   }
-  size_t want = round_size(bytes < (1u << 20) ? (1u << 20) : bytes);
-  RXW8_HIP(hipMalloc(&ws.ptr, want));
+  hipError_t e = hipMalloc(&ws.ptr, want);
+  if (e != hipSuccess && want > need) {
+    (void)hipGetLastError();
+    e = hipMalloc(&ws.ptr, want = need);
+  }
+  if (e != hipSuccess) {
+    ws.ptr = nullptr;
+    (void)hipGetLastError();
+    return hip_fail(e, "hipMalloc(&ws.ptr, want)");
+  }
   if (zero) {
     RXW8_HIP(hipMemsetAsync(ws.ptr, 0, want, rt->stream));
     RXW8_HIP(hipStreamSynchronize(rt->stream));
@@ -244,6 +262,7 @@ static void runtime_free(Runtime *rt) {
   for (auto &kv : rt->free_blocks) (void)hipFree(kv.second);
   for (Workspace *w : {&rt->partials, &rt->scratch, &rt->xcast, &rt->wdeq, &rt->attn_counters})
     if (w->ptr) (void)hipFree(w->ptr);
+  for (void *p : rt->retired) (void)hipFree(p);
   for (hipModule_t m : rt->modules) (void)hipModuleUnload(m);
   if (rt->own_stream) (void)hipStreamDestroy(rt->own_stream);
   delete static_cast<rxw8_runtime *>(rt);

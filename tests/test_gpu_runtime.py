@@ -56,3 +56,73 @@ def test_wrapped_torch_tensors_on_torch_stream(rt):
         assert float(np.abs(y.numpy() - ref).max() / np.abs(ref).max()) <= 1e-2
     finally:
         rt.set_stream(0)
+
+
+LINEARS = {  # kind: (rows, n, k, x, compute), a larger call of the same runtime, the splits of the mid-size GEMM
+    "mid-size splits": ((100, 2048, 6144, "bf16", "bf16"), (330, 4096, 6144, "bf16", "bf16"), "3"),
+    "bf16 copy of f32 rows": ((100, 1040, 512, "f32", "bf16"), (330, 1040, 4096, "f32", "bf16"), "1"),
+    "hi and lo parts": ((40, 1024, 2048, "f32", "f32"), (300, 1024, 2048, "f32", "f32"), "1"),
+    "gemv splits": ((8, 1024, 8192, "bf16", "bf16"), (16, 4096, 8192, "bf16", "bf16"), "1"),
+    "decode splits": (None, None, "1"),
+}
+
+
+@pytest.mark.parametrize("kind", list(LINEARS))
+def test_a_captured_call_outlives_its_workspaces(monkeypatch, kind):
+    """A caller's graph holds the addresses of the workspaces that its calls
+    used. A larger eager call replaces them; the replays still give the eager
+    result and touch nothing that was allocated since."""
+    import torch
+    import rxla_amd as rx
+
+    small, large, ks = LINEARS[kind]
+    monkeypatch.setenv("RXW8_MID_KS", ks)
+    own = rx.Runtime(0)
+    stream = torch.cuda.Stream()
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    keep = []
+
+    def linear(m, n, k, x, compute):
+        t = [rand(m, k).to(torch.bfloat16 if x == "bf16" else torch.float32),
+             torch.randint(1, 256, (n, k), generator=g, device="cuda", dtype=torch.uint8),
+             rand(n, k // 128).abs() * 1e-3, torch.empty(m, n, device="cuda")]
+        keep.append(t)
+        b = [own.wrap_tensor(v) for v in t]
+        dt = rx.DType.F32 if compute == "f32" else rx.DType.BF16
+        return lambda: rx.quantized_linear(own, *b[:3], dt, rx.DType.F32, out=b[3]), t[3]
+
+    def decode(batch, length):
+        t = [rand(batch, 64, 128), rand(batch, 8, length, 128).bfloat16(), rand(batch, 8, length, 128).bfloat16(),
+             torch.full((batch,), length, device="cuda", dtype=torch.int32), torch.empty(batch, 64, 128, device="cuda")]
+        keep.append(t)
+        b = [own.wrap_tensor(v) for v in t]
+        return lambda: rx.grouped_query_attention(own, *b[:4], out=b[4]), t[4]
+
+    (call, y), (bigger, _) = ((linear(*small), linear(*large)) if small else (decode(1, 600), decode(8, 4000)))
+    torch.cuda.synchronize()
+    own.set_stream(stream.cuda_stream)
+    call()
+    own.synchronize()
+    eager = y.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        call()
+    torch.cuda.synchronize()
+    bigger()
+    own.synchronize()
+    # whatever the runtime gave back is handed out again here
+    since = [own.zeros((1 << 18,), rx.DType.F32) for _ in range(8)]
+    guard = [torch.full((1 << s,), 3.0, device="cuda") for s in range(16, 25)]
+    for _ in range(3):
+        y.fill_(7.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager)
+        bigger()
+        own.synchronize()
+    assert all(bool((t == 3.0).all()) for t in guard)
+    assert all(not b.to_numpy().any() for b in since)
+    own.set_stream(None)
