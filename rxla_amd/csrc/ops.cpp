@@ -761,12 +761,15 @@ static int run_linear_f32_gemm(Runtime *rt, const float *x, const uint8_t *w, bo
                                const float *scale, float *y, int64_t M, int64_t N, int64_t K,
                                int64_t G, int y_mode) {
   if (!f32_gemm_applies(w, y, M, N, K, G)) return RXW8_UNIMPLEMENTED;
-  const F32MidPlan mp = plan_f32_mid(rt, M, N, K, G);
+  F32MidPlan mp = plan_f32_mid(rt, M, N, K, G);
+  // no room for the partials (a capture before the first eager call): one
+  // split where its scales fit in LDS, else the 256 x 128 tiles and their rule
+  if (mp.ks > 1 && ensure_workspace(rt, rt->partials, (size_t)(mp.ks * M * N) * 4, false))
+    mp.ks = f32_mid_lds(mp.fj, 1, K, G) * 2 <= rt->lds_max ? 1 : 0;
   if (mp.ks > 0) {
     uint16_t *xh, *xl;
     int rc = f32_gemm_operands(rt, M, K, &xh, &xl);
     if (rc) return rc;
-    if (mp.ks > 1 && (rc = ensure_workspace(rt, rt->partials, (size_t)(mp.ks * M * N) * 4, false))) return rc;
     SplitXArgs sx{x, xh, xl, M * K};
     if (x && (rc = launch(rt, "rxw8_gemm_split_x", dim3(grid_for(M * K / 4, 256, 4096)), dim3(256), sx)))
       return rc;
@@ -995,7 +998,9 @@ static int run_gemm_mid(Runtime *rt, MidPlan p, const void *x, int x_f32, const 
                         const float *s, void *y, int y_f32, int64_t M, int64_t N, int64_t K, int64_t G,
                         int y_mode) {
   const int64_t fj = std::min<int64_t>(4, (M + 15) / 16);
-  const bool xf = x_f32 && M <= 64;
+  // (f32 rows are converted in the kernel as well where there is no room for
+  // their bf16 copy, a capture before the first eager call: the same values)
+  const bool xf = x_f32 && (M <= 64 || ensure_workspace(rt, rt->xcast, (size_t)(M * K) * 2, false));
   int rc;
   // no room for the partials (a capture before the first eager call): one
   // split needs none
@@ -1004,7 +1009,6 @@ static int run_gemm_mid(Runtime *rt, MidPlan p, const void *x, int x_f32, const 
     p.ks = 1;
   }
   if (x_f32 && !xf) {
-    if ((rc = ensure_workspace(rt, rt->xcast, (size_t)(M * K) * 2, false))) return rc;
     CastArgs c{(const float *)x, (uint16_t *)rt->xcast.ptr, M * K};
     if ((rc = launch(rt, "rxw8_gemm_cast_x", dim3(grid_for(M * K / 4 + 1, 256, 4096)), dim3(256), c)))
       return rc;

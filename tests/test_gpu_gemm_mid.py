@@ -109,3 +109,52 @@ def test_f32_compute_tiles(rt, monkeypatch, m, n, k, g, ks, packed):
         wi = r.pack_weight(rt, wi)
     yi = r.quantized_linear(rt, rt.buffer(xi), wi, rt.buffer(si), r.DType.F32, r.DType.F32).to_numpy()
     np.testing.assert_array_equal(yi, xi.astype(np.float64) @ (ui.astype(np.float64) - 128).T)
+
+
+@pytest.mark.parametrize("m,n,k,x,compute,split", [
+    (100, 1040, 512, "f32", "bf16", False), (300, 1040, 512, "f32", "bf16", False),
+    (300, 2048, 4096, "bf16", "bf16", True), (17, 32768, 1024, "f32", "f32", True)])
+def test_a_first_call_in_a_capture(m, n, k, x, compute, split):
+    """A capture can't size a workspace. A call that comes first there, with no
+    room for the bf16 copy of its f32 rows, gives the eager bits; one with no
+    room for its K splits runs without them (the sums in another order: one
+    bf16 step, or 1e-5 in F32)."""
+    import torch
+    r = rx()
+    g = torch.Generator(device="cuda").manual_seed(m)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    t = [rand(m, k).to(torch.float32 if x == "f32" else torch.bfloat16),
+         torch.randint(1, 256, (n, k), generator=g, device="cuda", dtype=torch.uint8),
+         rand(n, k // 128).abs() * 1e-3, torch.zeros(m, n, device="cuda")]
+    torch.cuda.synchronize()
+    dt = r.DType.F32 if compute == "f32" else r.DType.BF16
+
+    def call(own, rows=m, chans=n):
+        b = [own.wrap_tensor(v) for v in (t[0][:rows], t[1][:chans], t[2][:chans])]
+        out = t[3][:rows, :chans] if chans == n else torch.empty(rows, chans, device="cuda")
+        return r.quantized_linear(own, *b, dt, r.DType.F32, out=own.wrap_tensor(out)), out
+
+    eager = r.Runtime(0)
+    call(eager)
+    eager.synchronize()
+    want = t[3].clone()
+    own, stream = r.Runtime(0), torch.cuda.Stream()
+    own.set_stream(stream.cuda_stream)
+    if compute == "f32":  # (its hi and lo parts need their buffer in any plan)
+        _, small = call(own, chans=64)
+        own.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="thread_local"):
+        call(own)
+    for _ in range(3):
+        t[3].fill_(7.0)
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        if not split:
+            assert torch.equal(t[3], want)
+        else:
+            step = 1e-5 if compute == "f32" else 2.0 ** -7
+            assert float(((t[3] - want).abs() / want.abs().clamp_min(want.std())).max()) <= step
+    own.set_stream(None)
