@@ -690,18 +690,13 @@ struct SplitXArgs {
   int64_t n;
 };
 
-// F32-compute W8 linear for long inputs on the GEMM tiles
-// (rxw8_gemm_f32c): x split into bf16 hi / lo parts in the runtime's
-// staging buffer, then 256 x 128 output tiles that read each weight tile
-// once per 128 rows of x. Shapes with fewer tiles than half a round of CUs
-// split K (at scale-group boundaries, at least 4 k tiles per split, up to 8
-// splits) toward a round of work items, and a reduce launch adds the
-// partials in split order. Taken from 17 rows on (RXW8_F32_GEMM=0 / 1
-// forces it off / on where it applies; RXW8_F32_GEMM_KSPLIT=n forces n
-// splits): even with mostly empty 128-row tiles and 32-64 work items it
-// beats the row kernels, which read the weights once per 32 rows and cut K
-// into LDS-sized launches (Qwen3.5-0.8B forward at 17 / 64 positions: 2.80
-// / 3.39 ms against 3.95 / 4.61); up to 16 rows the F32 GEMV stays.
+// F32-compute W8 linear from 17 rows on (up to 16 the F32 GEMV stays): x split
+// into bf16 hi / lo parts in the runtime's staging buffer, then GEMM tiles of
+// gemm_mid.hip or gemm.hip by plan_f32_mid. Even with mostly empty tiles they
+// beat the row kernels, which read the weights once per 32 rows and cut K into
+// LDS-sized launches (Qwen3.5-0.8B forward at 17 / 64 positions: 2.80 / 3.39
+// ms on the 256 x 128 tiles against 3.95 / 4.61). RXW8_F32_GEMM=0 / 1 forces
+// both off / on where they apply.
 // UNIMPLEMENTED (nothing launched) when the shape or the 16-byte alignment
 // of the weights and y does not fit its contract.
 bool f32_gemm_applies(const void *w, const float *y, int64_t M, int64_t N, int64_t K, int64_t G) {
@@ -719,14 +714,47 @@ int f32_gemm_operands(Runtime *rt, int64_t M, int64_t K, uint16_t **hi, uint16_t
   return RXW8_OK;
 }
 
+// K splits of the 256 x 128 tiles of gemm.hip (rxw8_gemm_f32c, each weight tile
+// read once per 128 rows of x): shapes with fewer tiles than half a round of
+// CUs split K (at scale-group boundaries, or between the k tiles of a single
+// group, at least 4 k tiles per split, up to 8 splits) toward a round of work
+// items, and a reduce launch adds the partials in split order.
+// RXW8_F32_GEMM_KSPLIT=n forces n splits of these tiles. `per`: k tiles of a
+// work item.
+static int64_t f32_tile_splits(const Runtime *rt, int64_t M, int64_t N, int64_t K, int64_t G, int64_t *per) {
+  const int64_t tiles = (M + 127) / 128 * ((N + 255) / 256);
+  const int64_t ng = K / G, units = ng > 1 ? ng : K / 64, upt = ng > 1 ? G / 64 : 1;
+  const int ks_env = env_int("RXW8_F32_GEMM_KSPLIT", 0);
+  int64_t ks = 1;
+  if (ks_env > 0) {
+    ks = std::min<int64_t>(ks_env, units);
+  } else if (2 * tiles < rt->cus) {
+    for (int c : {2, 3, 4, 6, 8}) {
+      if (units / c * upt < 4) break;
+      ks = c;
+      if (tiles * c >= rt->cus) break;
+    }
+  }
+  *per = (units + ks - 1) / ks * upt;
+  return ks;
+}
+
 // F32-compute tiles of 256 x 64 (or 32) with the weights in registers, two
 // workgroups per CU (kernels/gemm_mid.hip): tile rows / 16, and K splits by
 // the least modelled time (us per 128-k chunk of a workgroup alone on its CU
 // and of two sharing it, a split's reduce 2.5 plus its partials at 2.5 TB/s;
-// fitted to sweeps of 1 to 12 splits). ks 0 where they do not apply (K % 128);
-// elsewhere they beat or tie the 256 x 128 tiles of gemm.hip from 17 to 2048
-// rows: 500 x 7168 x 1024 47.8 -> 30.8 us, 330 x 8320 x 1024 45.2 -> 30.3, 17 x
-// 1024 x 3584 21.8 -> 14.5, 500 x 248320 x 1024 618 -> 603.
+// fitted to sweeps of 1 to 12 splits). ks 0 where they do not apply (K % 128).
+// Measured against the 256 x 128 tiles over 17 to 16384 rows, N 256 to 16384,
+// K 1024 to 8192, both layouts: they win or tie (within 4%) in one round of
+// workgroups (512) up to 4096 rows, and in any number of rounds without
+// splits (500 x 7168 x 1024 47.8 -> 30.8 us, 17 x 1024 x 3584 21.8 -> 14.5,
+// 16384 x 8192 x 1024 623 -> 545). But two workgroups' grouped scales fit in
+// LDS only up to about 16 groups of 256 rows, so that longer K splits also
+// where the rows fill the chip, and the partials then cost more than the
+// tiles gain (8192 x 1024 x 2048 90 -> 106, 2048 x 16384 x 2048 272 -> 346).
+// There the modelled times decide, in us, fitted to the same sweep within 5%:
+// what both spend, rounds x k per work item (less where a round is partly
+// empty), and partials at 4.5 and 4.8 TB/s.
 struct F32MidPlan {
   int fj = 4, ks = 0;
 };
@@ -734,7 +762,7 @@ static size_t f32_mid_lds(int64_t fj, int ks, int64_t K, int64_t G) {
   const int64_t span = (K / 128 + ks - 1) / ks * 128;
   return (size_t)(4 * 16 * fj * 256) + (size_t)((span + G - 1) / G + 1) * 256 * 4;
 }
-static F32MidPlan plan_f32_mid(const Runtime *rt, int64_t M, int64_t N, int64_t K, int64_t G) {
+static F32MidPlan plan_f32_mid(const Runtime *rt, int64_t M, int64_t N, int64_t K, int64_t G, bool packed) {
   F32MidPlan p;
   const int env = env_int("RXW8_F32_MID", 1), forced = env_int("RXW8_F32_MID_KS", 0);
   if (!env || K % 128 || K >= ((int64_t)1 << 22) || env_int("RXW8_F32_GEMM_KSPLIT", 0)) return p;
@@ -752,6 +780,20 @@ static F32MidPlan plan_f32_mid(const Runtime *rt, int64_t M, int64_t N, int64_t 
     if (ks > 1) us += 2.5 + (ks + 1.0) * (double)M * N * 4.0 / 2.5e6;
     if (p.ks == 0 || us < best) best = us, p.ks = ks;
   }
+  const int64_t wgs = tiles * p.ks, round = 2 * rt->cus;
+  if (p.ks == 0 || forced || env > 1 || (wgs <= round && M <= 4096) || (p.ks == 1 && wgs > round)) return p;
+  const double both = 10.9 + 1.23e-6 * (double)(M * K), mn = 4e-6 * (double)(M * N);
+  const int64_t per = (chunks + p.ks - 1) / p.ks, rounds = (wgs + round - 1) / round;
+  double mid = wgs <= rt->cus ? 2.05 * (double)per
+                              : 3.62 * (double)(rounds * per) * (0.3 + 0.7 * (double)wgs / (double)(rounds * round));
+  if (p.ks > 1) mid += (double)(p.ks + 1) * mn / 4.84;
+  int64_t tper = 0;
+  const int64_t tks = f32_tile_splits(rt, M, N, K, G, &tper);
+  const int64_t items = (M + 127) / 128 * ((N + 255) / 256) * tks, trounds = (items + rt->cus - 1) / rt->cus;
+  double big = 1.91 * (double)(trounds * tper) * (0.78 + 0.22 * (double)items / (double)(trounds * rt->cus));
+  if (tks > 1) big += (double)(tks + 1) * mn / 4.54;
+  // (row-major codes cost these tiles 3.5% and the others nothing)
+  if ((both + mid) * (packed ? 1.0 : 1.035) >= 0.98 * (both + big)) p.ks = 0;
   return p;
 }
 
@@ -761,7 +803,7 @@ static int run_linear_f32_gemm(Runtime *rt, const float *x, const uint8_t *w, bo
                                const float *scale, float *y, int64_t M, int64_t N, int64_t K,
                                int64_t G, int y_mode) {
   if (!f32_gemm_applies(w, y, M, N, K, G)) return RXW8_UNIMPLEMENTED;
-  F32MidPlan mp = plan_f32_mid(rt, M, N, K, G);
+  F32MidPlan mp = plan_f32_mid(rt, M, N, K, G, packed);
   // no room for the partials (a capture before the first eager call): one
   // split where its scales fit in LDS, else the 256 x 128 tiles and their rule
   if (mp.ks > 1 && ensure_workspace(rt, rt->partials, (size_t)(mp.ks * M * N) * 4, false))
@@ -784,19 +826,8 @@ static int run_linear_f32_gemm(Runtime *rt, const float *x, const uint8_t *w, bo
     return launch(rt, "rxw8_gemm_f32c_reduce", dim3(grid_for(M * N / 4, 256, 4096)), dim3(256), r);
   }
   const int64_t tiles = (M + 127) / 128 * ((N + 255) / 256);
-  // split units: scale groups, or the k tiles of a single group
-  const int64_t ng = K / G, units = ng > 1 ? ng : K / 64, upt = ng > 1 ? G / 64 : 1;
-  const int ks_env = env_int("RXW8_F32_GEMM_KSPLIT", 0);
-  int64_t ks = 1;
-  if (ks_env > 0) {
-    ks = std::min<int64_t>(ks_env, units);
-  } else if (2 * tiles < rt->cus) {
-    for (int c : {2, 3, 4, 6, 8}) {
-      if (units / c * upt < 4) break;
-      ks = c;
-      if (tiles * c >= rt->cus) break;
-    }
-  }
+  int64_t per = 0;
+  const int64_t ks = f32_tile_splits(rt, M, N, K, G, &per);
   uint16_t *xh, *xl;
   int rc = f32_gemm_operands(rt, M, K, &xh, &xl);
   if (rc) return rc;

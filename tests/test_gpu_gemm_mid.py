@@ -158,3 +158,35 @@ def test_a_first_call_in_a_capture(m, n, k, x, compute, split):
             step = 1e-5 if compute == "f32" else 2.0 ** -7
             assert float(((t[3] - want).abs() / want.abs().clamp_min(want.std())).max()) <= step
     own.set_stream(None)
+
+
+@pytest.mark.parametrize("m,n,k,compute,mid", [
+    (4096, 2048, 2048, "f32", False), (512, 16384, 2048, "f32", False), (2048, 3072, 3584, "f32", False),
+    (500, 7168, 1024, "f32", True), (300, 1024, 3584, "f32", True), (5000, 5120, 1024, "f32", True)])
+def test_default_route(rt, monkeypatch, m, n, k, compute, mid):
+    """Where the mid-size tiles measured slower than the kernels that they
+    stand beside, the default rule leaves the call to those: its bits are those
+    of the one path, and not those of the other (other orders of summation)."""
+    import torch
+    r = rx()
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
+    t = [rand(m, k), torch.randint(1, 256, (n, k), generator=g, device="cuda", dtype=torch.uint8),
+         rand(n, k // 128).abs() * 1e-3]
+    torch.cuda.synchronize()
+    dt = r.DType.F32 if compute == "f32" else r.DType.BF16
+    env = "RXW8_F32_MID" if compute == "f32" else "RXW8_GEMM_MID"
+    wb = r.pack_weight(rt, rt.wrap_tensor(t[1]))
+
+    def call(mode):
+        if mode:
+            monkeypatch.setenv(env, mode)
+        y = torch.empty(m, n, device="cuda")
+        torch.cuda.synchronize()
+        r.quantized_linear(rt, rt.wrap_tensor(t[0]), wb, rt.wrap_tensor(t[2]), dt, r.DType.F32, out=rt.wrap_tensor(y))
+        rt.synchronize()
+        return y
+
+    default, without, forced = call(None), call("0"), call("2")
+    assert not torch.equal(without, forced)
+    assert torch.equal(default, forced if mid else without)
