@@ -410,6 +410,14 @@ static GemvPlan plan_gemv(const Runtime *rt, int64_t m, int64_t n, int64_t k, in
   return p;
 }
 
+// Whether a plain call asks plan_gemv for the wide single-launch tilings
+static bool gemv_prefers_one_launch(const Runtime *rt, int64_t M, int64_t N, int64_t K, bool w_bf16, bool ref_cast) {
+  const int wide_env = env_int("RXW8_GEMV_PREFER_WIDE", -1);
+  return wide_env >= 0 ? wide_env != 0
+                       : (!w_bf16 && ((N / 64 >= rt->cus && !(ref_cast && M == 1)) ||
+                                      (M >= 8 && N * K <= 17000000)));
+}
+
 static bool is_f(int dt) { return dt == RXW8_F32 || dt == RXW8_BF16; }
 
 // y[M, N] = linear(x[M, K]) on the GEMV kernel in chunks of <= 32 rows, with an
@@ -433,11 +441,7 @@ static int run_gemv(Runtime *rt, const void *x, int x_f32, const void *w, bool w
   // of 16 rows for N = 24576, streams faster than the wide tiles, 18.4
   // against 18.8 us; from 4 rows on the wide tiles win)
   GemvOptions plain;
-  const int wide_env = env_int("RXW8_GEMV_PREFER_WIDE", -1);
-  plain.prefer_ks1 =
-      wide_env >= 0 ? wide_env != 0
-                    : (!w_bf16 && ((N / 64 >= rt->cus && !(ref_cast && M == 1)) ||
-                                   (M >= 8 && N * K <= 17000000)));
+  plain.prefer_ks1 = gemv_prefers_one_launch(rt, M, N, K, w_bf16, ref_cast);
   if (!pro) pro = &plain;
   // Activations as MFMA fragments from global memory (XG) paid off for the
   // exact-code kernels when the weights are small next to the staging each
@@ -988,6 +992,7 @@ struct MidPlan {
   int rg = 0, ks = 1;
   double us = 1e30;
 };
+static const double kMidStep[2][4] = {{0.9, 1.4, 1.45, 1.85}, {1.6, 2.3, 2.7, 3.3}};  // [rg - 1][fj - 1]
 // LDS of a workgroup: two buffers of 16 fj x 256 bf16 of x per wave group, and
 // the grouped scales of one split (the most groups that ceil(chunks / ks)
 // chunks can touch)
@@ -1002,14 +1007,13 @@ static bool mid_applies(const void *x, const void *w, const void *y, int64_t M, 
          !env_int("RXW8_FORCE_GENERIC", 0);
 }
 static MidPlan plan_mid(const Runtime *rt, int64_t M, int64_t N, int64_t K, int64_t G, int x_f32, int y_mode) {
-  static const double step[2][4] = {{0.9, 1.4, 1.45, 1.85}, {1.6, 2.3, 2.7, 3.3}};
   const int64_t fj = std::min<int64_t>(4, (M + 15) / 16), chunks = K / 256;
   const int forced_rg = env_int("RXW8_MID_RG", 0), forced_ks = env_int("RXW8_MID_KS", 0);
   MidPlan p;
   for (int rg : {1, 2}) {
     if (forced_rg && rg != forced_rg) continue;
     const int64_t tiles = (M + 16 * fj - 1) / (16 * fj) * ((N + 64 * rg - 1) / (64 * rg));
-    double tau = step[rg - 1][fj - 1] * (G == K ? 1.0 : 1.1);
+    double tau = kMidStep[rg - 1][fj - 1] * (G == K ? 1.0 : 1.1);
     if (x_f32 && M <= 64) tau *= 1.25;
     for (int ks : {1, 2, 3, 4, 6, 8, 12, 16}) {
       if (ks > 1 && (2 * ks > chunks || y_mode == 2)) break;
@@ -1024,6 +1028,33 @@ static MidPlan plan_mid(const Runtime *rt, int64_t M, int64_t N, int64_t K, int6
     }
   }
   return p;
+}
+// Up to 32 rows, where the GEMV has a one-launch tiling: whether that is the
+// faster one. plan_mid's model and the GEMV's line below it are too coarse
+// there (8 x 4096 x 1024, f32 rows: 4.3 us of GEMV against 6.2). Both times in
+// us, fitted (within 8 and 6%) to 3000 calls of 5 to 32 rows, N 256 to 24576, K
+// 256 to 12288, replayed from a graph: the GEMV's loads by latency (64-k slices
+// of a wave) or by bytes, and x staged by each workgroup; the mid-size GEMM as
+// plan_mid has it. The mid-size GEMM has to win by 5%. Not asked beyond 16
+// rows of at least 64 channels per CU, where plan_mid's line decides better.
+static bool one_launch_gemv_wins(const Runtime *rt, const MidPlan &p, int64_t M, int64_t N, int64_t K, int64_t G,
+                                 int x_f32, bool packed) {
+  if (M > 32 || (M > 16 && N / 64 >= rt->cus)) return false;
+  const char *rc_env = std::getenv("RXW8_GEMV_REF_CAST");
+  const bool one = gemv_prefers_one_launch(rt, M, N, K, false, !(rc_env && *rc_env == '0'));
+  const GemvPlan g = plan_gemv(rt, std::min<int64_t>(M, M <= 16 ? 16 : 32), N, K, G, false, one);
+  if (g.ks != 1) return false;
+  const double rounds = (double)(((N + 16 * g.rw - 1) / (16 * g.rw) + rt->cus - 1) / rt->cus);
+  const double lat = 0.21 * rounds * (double)(K * g.rw / g.nw / 64);
+  const double bytes = 0.125e-6 * (double)(N * K) * (packed ? 1.0 : 1.45) * (G == K ? 1.0 : 1.22);
+  const double gemv = 3.2 + std::sqrt(std::sqrt(lat * lat * lat * lat + bytes * bytes * bytes * bytes)) +
+                      0.69 * rounds * (double)(M * K) / 16384.0 * (x_f32 ? 1.62 : 1.0);
+  const int64_t fj = (M + 15) / 16, tiles = (N + 64 * p.rg - 1) / (64 * p.rg);
+  const double tau = kMidStep[p.rg - 1][fj - 1] * (G == K ? 1.0 : 1.22) * (x_f32 ? 1.25 : 1.0);
+  double mid = (double)((tiles * p.ks + rt->cus - 1) / rt->cus) *
+               ((double)((K / 256 + 2 * p.ks - 1) / (2 * p.ks)) * tau * 1.04 + 2.62);
+  if (p.ks > 1) mid += 1.95 + (p.ks + 1.0) * (double)(M * N) * 4.0 / 1.86e6;
+  return mid * (packed ? 1.0 : 1.1) >= 0.95 * gemv;
 }
 static int run_gemm_mid(Runtime *rt, MidPlan p, const void *x, int x_f32, const uint8_t *w, bool packed,
                         const float *s, void *y, int y_f32, int64_t M, int64_t N, int64_t K, int64_t G,
@@ -1193,7 +1224,8 @@ int qlinear_launch(Runtime *rt, const void *x, int x_f32, const uint8_t *w, bool
     const double gemv = M <= 16 ? 7.0 + 0.24 * mb
                                 : (double)((M + 31) / 32) * (x_f32 ? 5.0 + 0.45 * mb : 4.0 + 0.42 * mb);
     const MidPlan p = plan_mid(rt, M, N, K, G, x_f32, y_mode);
-    if (p.rg && (p.us < gemv || env_int("RXW8_GEMM_MID", 1) > 1)) {
+    if (p.rg && ((p.us < gemv && !one_launch_gemv_wins(rt, p, M, N, K, G, x_f32, packed)) ||
+                 env_int("RXW8_GEMM_MID", 1) > 1)) {
       const int rc = run_gemm_mid(rt, p, x, x_f32, w, packed, s, y, y_f32, M, N, K, G, y_mode);
       if (rc != RXW8_UNIMPLEMENTED) return rc;
     }

@@ -161,6 +161,8 @@ def test_a_first_call_in_a_capture(m, n, k, x, compute, split):
 
 
 @pytest.mark.parametrize("m,n,k,compute,mid", [
+    (8, 4096, 1024, "bf16", False), (16, 2048, 2048, "bf16", False), (6, 24576, 1536, "bf16", False),
+    (12, 12288, 2048, "bf16", True), (48, 2048, 2048, "bf16", True),
     (4096, 2048, 2048, "f32", False), (512, 16384, 2048, "f32", False), (2048, 3072, 3584, "f32", False),
     (500, 7168, 1024, "f32", True), (300, 1024, 3584, "f32", True), (5000, 5120, 1024, "f32", True)])
 def test_default_route(rt, monkeypatch, m, n, k, compute, mid):
