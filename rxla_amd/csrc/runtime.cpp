@@ -289,8 +289,15 @@ int rxw8_status_is_retryable(int status) {
 int rxw8_abi_version(void) { return RXW8_ABI_VERSION; }
 
 // The f32 attention blocks of the loaded code object, their counters cleared
-// and waited for on the runtime's own new stream.
+// and waited for on the runtime's own new stream. (In relaxed capture mode: a
+// capture that this or another thread has in progress elsewhere would refuse
+// the calls, which do not touch its stream.)
 static int f32_attention_setup(Runtime *rt) {
+  struct Relaxed {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~Relaxed() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  } relaxed;
   hipDeviceptr_t p = nullptr;
   size_t bytes = 0;
   RXW8_HIP(hipModuleGetGlobal(&p, &bytes, rt->modules[(size_t)module_of("rxw8_gqa_tile_")],

@@ -126,3 +126,48 @@ def test_a_captured_call_outlives_its_workspaces(monkeypatch, kind):
     assert all(bool((t == 3.0).all()) for t in guard)
     assert all(not b.to_numpy().any() for b in since)
     own.set_stream(None)
+
+
+@pytest.mark.parametrize("mode", ["thread_local", "global"])
+@pytest.mark.parametrize("same_thread", [True, False])
+def test_a_runtime_is_created_beside_a_capture(mode, same_thread):
+    """While a stream is being captured, by this thread or another one, a
+    runtime can be created (loading its kernels may end that capture: HIP's
+    own rule), and its split attention works once the capture is over."""
+    import threading
+
+    import torch
+    import rxla_amd as rx
+
+    made, stream = [], torch.cuda.Stream()
+    x = torch.zeros(4, device="cuda")
+
+    def make():
+        try:
+            made.append(rx.Runtime(0))
+        except rx.Error as e:
+            made.append(e)
+
+    torch.cuda.synchronize()
+    try:
+        with torch.cuda.graph(torch.cuda.CUDAGraph(), stream=stream, capture_error_mode=mode):
+            x += 1
+            if same_thread:
+                make()
+            else:
+                t = threading.Thread(target=make)
+                t.start()
+                t.join()
+    except RuntimeError:
+        pass
+    torch.cuda.synchronize()
+    assert isinstance(made[0], rx.Runtime), made[0]
+    own, rng = made[0], np.random.default_rng(4)
+    q, k, v = (rng.standard_normal(s).astype(np.float32) for s in ((1, 4, 256), (1, 2, 600, 256), (1, 2, 600, 256)))
+    out = [rx.grouped_query_attention(own, own.buffer(q), own.buffer(k), own.buffer(v),
+                                      own.buffer(np.array([600], np.int32))).to_numpy() for _ in range(3)]
+    s = np.einsum("hgd,hkd->hgk", q[0].reshape(2, 2, 256).astype(np.float64), k[0]) / 16
+    p = np.exp(s - s.max(-1, keepdims=True))
+    want = np.einsum("hgk,hkd->hgd", p / p.sum(-1, keepdims=True), v[0].astype(np.float64)).reshape(4, 256)
+    for o in out:
+        assert np.abs(o[0] - want).max() <= 1e-5
