@@ -90,9 +90,15 @@ def test_decoder_prefill_and_decode_match_oracle(rt, group):
     np.testing.assert_array_equal(model.lens()[:batch], [12, 12])
 
 
-def test_decoder_long_prefill_matches_oracle(rt):
-    """2 x 40 prompt rows: every projection of the prefill runs on the M > 64
-    GEMM, including the residual (h += bf16(o_proj), h += bf16(down)) epilogue."""
+@pytest.mark.parametrize("mid,rg,ks", [("1", "0", "0"), ("0", "0", "0"), ("2", "1", "1"), ("2", "1", "2"),
+                                       ("2", "2", "1"), ("2", "2", "2")])
+def test_decoder_long_prefill_matches_oracle(rt, monkeypatch, mid, rg, ks):
+    """2 x 40 prompt rows: every projection of the prefill runs on a GEMM,
+    including the residual (h += bf16(o_proj), h += bf16(down)) and SwiGLU
+    epilogues: by the default rule, on the 128-row tiles, and on the mid-size
+    tiles of 64 and 128 channels without and (K = 1024: down) with a K split."""
+    for name, value in (("RXW8_GEMM_MID", mid), ("RXW8_MID_RG", rg), ("RXW8_MID_KS", ks)):
+        monkeypatch.setenv(name, value)
     cfg = small_cfg(max_seq=48, group=128)
     params = tiny_params(cfg, seed=81, std=0.05)
     batch = 2
