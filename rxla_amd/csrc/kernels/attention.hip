@@ -1130,31 +1130,6 @@ __device__ void attn_prefill_wh(const PrefillArgs &a) {
   }
 }
 
-typedef __attribute__((address_space(3))) void lds_void;
-
-// One LDS DMA instruction of the wave: lane l copies 16 bytes from g (its own
-// address) to LDS at l_base + 16 l (l_base wave-uniform); completion is
-// counted by vmcnt.
-__device__ __forceinline__ void lds_dma16(const void *g, void *l_base) {
-  __builtin_amdgcn_global_load_lds(g, (lds_void *)l_base, 16, 0, 0);
-}
-
-// The same copy from inline asm, base + voff (base wave-uniform in SGPRs, byte
-// offset per lane) into LDS at lds + 16 l: the compiler then does not answer
-// LDS reads of the other buffer with waits on the copy (the caller waits
-// before the barrier that publishes it).
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void lds_dma16_asm(const void *base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2"
-               :: "v"(voff), "s"(lds), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-__device__ __forceinline__ uint32_t lds_u32(const uint16_t *p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint16_t *)p;
-}
-
 // (constant arguments of the generic lambdas below)
 struct Yes { static constexpr bool value = true; };
 struct No { static constexpr bool value = false; };
@@ -1223,19 +1198,19 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
   const uint32_t kx = (uint32_t)((lane & 15) ^ (drow & 15)) << 4;
   const uint32_t vx = (uint32_t)((lane & 15) ^ (2 * (drow & 7))) << 4;
   auto dma_k = [&](int blk) {
-    const uint32_t dst = lds_u32(k_lds0 + (blk & (NB - 1)) * PKB * D) + 1024 * wv;
+    const uint32_t dst = lds_addr(k_lds0 + (blk & (NB - 1)) * PKB * D) + 1024 * wv;
 #pragma unroll
     for (int n = 0; n < 4 / HW; ++n) {
       const int key = min(blk * PKB + drow + 16 * HW * n, kv_end - 1);
-      lds_dma16_asm(a.kc + kv_base, (uint32_t)key * (2 * D) + kx, dst + 4096 * HW * n);
+      dma16(a.kc + kv_base, (uint32_t)key * (2 * D) + kx, dst + 4096 * HW * n);
     }
   };
   auto dma_v = [&](int blk) {
-    const uint32_t dst = lds_u32(v_lds0 + (blk & (NB - 1)) * PKB * D) + 1024 * wv;
+    const uint32_t dst = lds_addr(v_lds0 + (blk & (NB - 1)) * PKB * D) + 1024 * wv;
 #pragma unroll
     for (int n = 0; n < 4 / HW; ++n) {
       const int key = min(blk * PKB + drow + 16 * HW * n, kv_end - 1);
-      lds_dma16_asm(a.vc + kv_base, (uint32_t)key * (2 * D) + vx, dst + 4096 * HW * n);
+      dma16(a.vc + kv_base, (uint32_t)key * (2 * D) + vx, dst + 4096 * HW * n);
     }
   };
   // what the first block needs goes out before anything else (q's loads
@@ -1316,8 +1291,8 @@ __device__ void attn_prefill_rt(const PrefillArgs &a) {
   const int tr_j = col >> 2, tr_q = col & 3;
   // LDS byte addresses of the fragments: one XOR and a constant offset from
   // these (chunk 4 t + g4 of K row col, values 16 dt + 4 tr_q of V row 4 g4 + tr_j)
-  uint32_t k_frag0 = lds_u32(k_lds0) + 2 * col * D + ((g4 ^ col) << 4);
-  uint32_t v_frag0 = lds_u32(v_lds0) + 2 * (4 * g4 + tr_j) * D +
+  uint32_t k_frag0 = lds_addr(k_lds0) + 2 * col * D + ((g4 ^ col) << 4);
+  uint32_t v_frag0 = lds_addr(v_lds0) + 2 * (4 * g4 + tr_j) * D +
                      ((2 * ((4 * g4 + tr_j) & 7)) << 4) + ((tr_q & 1) << 3);
   v_frag0 ^= (tr_q >> 1) << 4;
   auto k_frag = [&](uint32_t base, int kt, int t) {

@@ -83,25 +83,14 @@ __device__ __forceinline__ float max4(float v) {
 }
 __device__ __forceinline__ float sum4(float v) { return sum_xor32(sum_xor16(v)); }
 
-// 16 bytes per lane, base + voff -> LDS at lds + 16 * lane (base and lds
-// wave-uniform). From inline asm: the compiler then does not answer LDS reads
-// of the other buffer with waits on it; the loop itself waits before the
-// barrier that publishes a tile.
+// 4 bytes per lane from the lane's own address to LDS at lds + 4 * lane (see dma16)
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma16(const void *base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2"
-               :: "v"(voff), "s"(lds), "s"(base) : "memory", "m0");
-}
-// 4 bytes per lane from the lane's own address to LDS at lds + 4 * lane
 __device__ __forceinline__ void dma4(const float *p, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dword %0, off"
                :: "v"(p), "s"(lds) : "memory", "m0");
 }
 #pragma clang diagnostic pop
-__device__ __forceinline__ uint32_t lds_addr(const char *p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
-}
 
 // K / V elements: ES bytes each, EPC per 16-byte piece
 template <bool BF>
@@ -301,6 +290,11 @@ __device__ __forceinline__ void load_q(const GqaTileArgs &a, int64_t at, int j, 
 
 // e^(s - m); before any visible key (m = -inf) every score is -inf and weighs
 // nothing, or is NaN and stays it.
+// (__expf rounds (s - m) log2(e), an error that grows with |s - m| but stays
+// below that of the score itself. Against 64 bits, at widths 64 / 128 / 256, 1
+// and 200 queries, 700 keys, scores of width 1 to 64: 1.8e-7 to 1.9e-6 with it
+// where the scalar kernels with expf give 5.1e-7 to 8.1e-6; equal, 1e-6 to
+// 4.5e-6 on both, with 200 added to every score.)
 __device__ __forceinline__ float prob(float s, float m) {
   return m == kNegInf ? (s != s ? s : 0.f) : __expf(s - m);
 }
@@ -622,7 +616,7 @@ __device__ void gqa_tile(const GqaTileArgs &a) {
 // first tile, merge): 4 x 8 / 2 heads, D = 256, f32, lengths 300-2048: 15.4 us
 // against 517 us for one workgroup per query head with scalar loads.
 template <int CB, int AB>
-__device__ __forceinline__ f32x4 mfma4(float x, float y, f32x4 c) {
+__device__ __forceinline__ f32x4 mfma4x4(float x, float y, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(x, y, c, CB, AB, 0);
 }
 template <int CTRL>
@@ -760,7 +754,7 @@ __device__ void gqa_quad(const GqaTileArgs &a) {
           for (int kq = 0; kq < 4; ++kq) {
             float kx;
             if constexpr (EPK == EPC) kx = T::el(kf[kq][i], e); else kx = T::four(kf[kq][i], e);
-            acc[s][kq] = mfma4<0, 0>(kx, qr[s][i * EPK + e], acc[s][kq]);
+            acc[s][kq] = mfma4x4<0, 0>(kx, qr[s][i * EPK + e], acc[s][kq]);
           }
       }
     const int tn = min(t + NW, t1 - 1);  // (the last tile is read again rather than branched over)
@@ -809,7 +803,7 @@ __device__ void gqa_quad(const GqaTileArgs &a) {
 #pragma unroll
         for (int e = 0; e < EPC; ++e)
 #pragma unroll
-          for (int s = 0; s < NS; ++s) o[s][e] = mfma4<CB, X>(p[s], T::el(vf[X], e), o[s][e]);
+          for (int s = 0; s < NS; ++s) o[s][e] = mfma4x4<CB, X>(p[s], T::el(vf[X], e), o[s][e]);
       });
     } else {
 #pragma unroll

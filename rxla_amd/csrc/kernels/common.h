@@ -105,6 +105,26 @@ __device__ __forceinline__ float wave_sum64(float v) {
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
+// global -> LDS DMA of 16 bytes per active lane (global_load_lds_dwordx4): lane
+// l copies from base + voff (base wave-uniform, byte offset per lane) to LDS
+// bytes [lds + 16 l, +16). Issued from inline asm on purpose: the compiler
+// models the builtin as a flat access of both global memory and LDS and then
+// answers every later LDS or VGPR-load dependency with lgkmcnt(0) / vmcnt(0),
+// which serialises the fragment reads with the MFMAs. The kernels wait for the
+// copied data themselves (explicit vmcnt before the barrier that publishes
+// it); the compiler, not knowing these loads, can only over-wait for its own.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
+__device__ __forceinline__ void dma16(const void *base, uint32_t voff, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2"
+               :: "v"(voff), "s"(lds), "s"(base) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+// The LDS byte address of a pointer into LDS
+__device__ __forceinline__ uint32_t lds_addr(const void *p) {
+  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
+}
+
 // Raw buffer resource over [base, base + bytes) (stride 0; the gfx9 word 3
 // with a 32-bit data format): a raw buffer load at a byte offset whose
 // access reaches past `bytes` returns zeros and reads no memory.

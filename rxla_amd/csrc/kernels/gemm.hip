@@ -61,26 +61,6 @@ constexpr int TN = 128, BK = 64, GROUP_N = 8;
 #define RXW8_GEMM_PREFETCH 2
 #endif
 
-// global -> LDS DMA of 16 bytes per lane (global_load_lds_dwordx4; lane l
-// writes LDS bytes [lds + 16 l, +16)). Issued from inline asm on purpose: the
-// compiler models the builtin as a flat access of both global memory and LDS
-// and then answers every later LDS or VGPR-load dependency with lgkmcnt(0) /
-// vmcnt(0), which serialises the fragment reads with the MFMAs. The kernels
-// wait for the DMA'd data themselves (explicit vmcnt before each barrier); the
-// compiler, not knowing these loads, can only over-wait for its own.
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void dma16(const void *base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2"
-               :: "v"(voff), "s"(lds), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-__device__ __forceinline__ uint32_t lds_addr(const char *p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
-}
-
-
 // Byte offset of 16-byte chunk c (0..7) of row r in a swizzled 128-B-row tile.
 __device__ __forceinline__ int swz(int r, int c) { return r * 128 + ((c ^ (r & 7)) << 4); }
 

@@ -43,20 +43,6 @@ namespace {
 constexpr int CK = 256;  // k per chunk
 constexpr int ROWB = CK * 2;
 
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-// global -> LDS DMA of 16 bytes per lane from inline asm: the compiler then
-// does not answer LDS reads of the other buffer with waits on it (the loop
-// waits before the barrier that publishes a chunk)
-__device__ __forceinline__ void dma16(const void *base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2"
-               :: "v"(voff), "s"(lds), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-__device__ __forceinline__ uint32_t lds_addr(const char *p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) char *)p;
-}
-
 // lane holds y[m, n .. n+3] (see gemm.hip gemm_store)
 __device__ __forceinline__ void store4(const GemmArgs &a, int m, int n, f32x4 v) {
   if (a.y_mode == 2) {
@@ -90,8 +76,9 @@ __device__ __forceinline__ void store4(const GemmArgs &a, int m, int n, f32x4 v)
   }
 }
 
-template <int FJ, int RG, int KG, bool GRP, bool XF>
+template <int FJ, int RG, bool GRP, bool XF>
 __device__ __forceinline__ void gemm_mid(const GemmArgs &a) {
+  constexpr int KG = 2;  // wave groups
   constexpr int TM = 16 * FJ, TN = 64 * RG, XBUF = TM * ROWB;
   constexpr int XDMA = XBUF / 1024 / 4;  // LDS-DMA instructions per wave per chunk
   extern __shared__ __attribute__((aligned(1024))) char smem[];
@@ -106,7 +93,7 @@ __device__ __forceinline__ void gemm_mid(const GemmArgs &a) {
   const int t_all = (int)(blockIdx.x % 8) * per_xcd + (int)(blockIdx.x / 8);
   if (t_all >= ntiles * a.ksplit) return;
   const int split = t_all / ntiles, t = t_all - split * ntiles;
-  constexpr int GN = RG >= 4 ? 4 : 8;
+  constexpr int GN = 8;
   const int group = t / (GN * tiles_m), in = t - group * GN * tiles_m, gw = min(GN, tiles_n - group * GN);
   const int n0 = (group * GN + in % gw) * TN + wn * 16 * RG, m0 = in / gw * TM;
   const int KT = a.K / 64, chunks = a.K / CK, groups = a.K / a.G;
@@ -165,7 +152,7 @@ __device__ __forceinline__ void gemm_mid(const GemmArgs &a) {
   float *scl = (float *)(smem + 2 * KG * XBUF);
   const uint32_t gk = (uint32_t)a.G / 64, ginv = gk > 1 ? 0xffffffffu / gk + 1 : 0;
   auto group_of = [&](int step) { return (int)(gk > 1 ? __umulhi((uint32_t)step, ginv) : (uint32_t)step); };
-  const int g_lo = GRP ? group_of(4 * cb) : 0, g_n = GRP ? group_of(4 * ce - 1) + 1 - g_lo : 0;
+  const int g_lo = GRP ? group_of(4 * cb) : 0, g_n = GRP ? group_of(4 * ce - 1) + 1 - g_lo : 1;
   auto stage_scales = [&]() {
     const int nt = n0 - wn * 16 * RG;  // the workgroup's first weight row
     for (int e = threadIdx.x; e < TN * g_n; e += 256 * KG) {
@@ -213,7 +200,7 @@ __device__ __forceinline__ void gemm_mid(const GemmArgs &a) {
     if constexpr (XF) load_x(cn);
     else issue_x(cn, (i + 1) & 1);
     load_w(cn, nxt);
-    const bool live = KG == 1 || cb + kg + KG * i < ce;  // (wave-uniform) this group has a chunk left
+    const bool live = cb + kg + KG * i < ce;  // (wave-uniform) this group has a chunk left
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       if (!live) break;
@@ -256,23 +243,19 @@ __device__ __forceinline__ void gemm_mid(const GemmArgs &a) {
   }
   if (i < iters) step(i, w0, w1);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the copies past the last chunk
-  if constexpr (KG > 1) {
-    __syncthreads();
-    f32x4 *red = (f32x4 *)smem;
-    if (kg > 0)
+  __syncthreads();
+  f32x4 *red = (f32x4 *)smem;
+  if (kg > 0)
 #pragma unroll
-      for (int g = 0; g < RG; ++g)
+    for (int g = 0; g < RG; ++g)
 #pragma unroll
-        for (int j = 0; j < FJ; ++j) red[(((kg - 1) * 4 + wn) * RG * FJ + g * FJ + j) * 64 + lane] = acc[g][j];
-    __syncthreads();
-    if (kg > 0) return;
+      for (int j = 0; j < FJ; ++j) red[(wn * RG * FJ + g * FJ + j) * 64 + lane] = acc[g][j];
+  __syncthreads();
+  if (kg > 0) return;
 #pragma unroll
-    for (int x = 0; x < KG - 1; ++x)
+  for (int g = 0; g < RG; ++g)
 #pragma unroll
-      for (int g = 0; g < RG; ++g)
-#pragma unroll
-        for (int j = 0; j < FJ; ++j) acc[g][j] += red[((x * 4 + wn) * RG * FJ + g * FJ + j) * 64 + lane];
-  }
+    for (int j = 0; j < FJ; ++j) acc[g][j] += red[(wn * RG * FJ + g * FJ + j) * 64 + lane];
   // lane holds D[n = 16 g + 4 kq + e][m = 16 j + r16]
 #pragma unroll
   for (int j = 0; j < FJ; ++j)
@@ -456,7 +439,7 @@ __device__ __forceinline__ void gemm_f32m(const LinearF32GemmArgs &a) {
 #define RXW8_GEMM_MID(FJ, RG, GRP, XF, SUFFIX)                                                   \
   extern "C" __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2)))      \
       rxw8_gemm_mid_m##FJ##_r##RG##SUFFIX(GemmArgs a) {                                          \
-    gemm_mid<FJ, RG, 2, GRP, XF>(a);                                                             \
+    gemm_mid<FJ, RG, GRP, XF>(a);                                                             \
   }
 #define RXW8_GEMM_MID_FJ(FJ)                 \
   RXW8_GEMM_MID(FJ, 1, false, false, )       \

@@ -333,21 +333,6 @@ __device__ __forceinline__ float row_add16(float v) {
   return v + dpp_rot<0xb1>(v);
 }
 
-// global -> LDS DMA of 16 bytes per active lane (global_load_lds_dwordx4:
-// lane l writes LDS bytes [lds + 16 l, +16)), from inline asm so the compiler
-// does not answer later LDS reads with waits on it (the caller waits).
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void q35_dma16(const void *base, uint32_t voff, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, %2"
-               :: "v"(voff), "s"(lds), "s"(base) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-
-__device__ __forceinline__ uint32_t q35_lds_addr(const float *p) {
-  return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) float *)p;
-}
-
 template <int D>
 __device__ void q35_attention(const Q35AttnArgs &a) {
   constexpr int DC = D / 4, DT = D / 16, KS = D + 4, PS = 20;
@@ -396,8 +381,8 @@ __device__ void q35_attention(const Q35AttnArgs &a) {
       for (int i = 0; i < 8; ++i) {
         const int row = wvu * 8 + i, kv = row >> 4, kr = row & 15;
         const int key = min(16 * t + kr, a.S - 1);
-        q35_dma16(kv ? vbase : kbase, (uint32_t)(key * D + 4 * lane) * 4u,
-                  q35_lds_addr(attn_lds + (2 * buf + kv) * TILE + kr * KS));
+        dma16(kv ? vbase : kbase, (uint32_t)(key * D + 4 * lane) * 4u,
+                  lds_addr(attn_lds + (2 * buf + kv) * TILE + kr * KS));
       }
     }
   };
