@@ -358,7 +358,7 @@ def bench_prefill_attention(rt, rx, torch, stream, reps=10):
     tf = flops / t / 1e12
     return {"bound": "mfma", "achieved": round(tf, 1), "peak": MFMA_BF16_PEAK_TFLOPS,
             "unit": "TFLOP/s", "frac": round(tf / MFMA_BF16_PEAK_TFLOPS, 4), "traffic": None,
-            "kernel": "rxw8_gqa_prefill_r2_d128_g2", "us_per_call": round(t * 1e6, 1),
+            "kernel": "rxw8_gqa_prefill_r2q32_d128_g2", "us_per_call": round(t * 1e6, 1),
             "flops_per_call": flops, "shape": "B=8 S=1024 Hq=16 Hkv=8 D=128, causal from 0",
             "note": "flops count the visible (causal) keys once; q enters as bf16 hi + lo, "
                     "so the MFMA work is 1.5x this count",
@@ -544,7 +544,7 @@ def bench_f32_linear(rt, rx, torch, stream, reps=10, n=248320, k=1024, g=128):
     del x, y, pk
     del ws
     return {"kernel": "rxw8_linear_f32_mfma_r1_w8 (S 16, row-major) / rxw8_linear_f32_mfma_pk_r1_w8 "
-                      "(S16_packed, tile layout) / rxw8_gemm_split_x + rxw8_gemm_f32c (S 1024)",
+                      "(S16_packed, tile layout) / rxw8_gemm_split_x + rxw8_gemm_mid_f32_m4 (S 1024)",
             "shape": f"W [{n}, {k}] U8, G {g} (the Qwen3.5-0.8B tied LM head), x F32 [S, {k}]",
             "runs": out,
             "note": "mfma_frac counts the hi and lo MFMAs (twice the algorithmic flops)",
