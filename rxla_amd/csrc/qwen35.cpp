@@ -622,18 +622,19 @@ int linear_mixer(Qwen35 *m, const Layer &L, int64_t B, int64_t S) {
     return out_proj(m, L, L.out, m->gated, m->f32c, T);
   }
   // conv + SiLU, q / k L2 norms, beta and decay: one workgroup per (token, head)
-  // Sequences of 256 positions or more, single ones of 160 (Dl 64 / 128), take
-  // the chunked delta rule: the chunks' triangular solves in parallel, then one
-  // walk over the chunks per 16 state columns on the matrix cores
-  // (RXW8_Q35_CHUNKED=0 / 1 forces it off / on). Its chunk pass costs ~17 us
-  // per layer whatever the length, the walk ~4 us per 64 positions, the
-  // sequential kernel ~0.2 us per position. The 0.8B forward at batch 1,
-  // sequential against chunked: 128 positions 3.12 / 3.15 ms, 160 3.47 / 3.41,
-  // 224 4.11 / 3.87, 256 4.26 / 3.89. (Between 160 and 256 a batch is not
-  // measured.)
+  // Sequences of 160 positions or more (Dl 64 / 128) take the chunked delta
+  // rule: the chunks' triangular solves in parallel, then one walk over the
+  // chunks per 16 state columns on the matrix cores (RXW8_Q35_CHUNKED=0 / 1
+  // forces it off / on). Its chunk pass costs ~17 us per layer whatever the
+  // length, the walk ~4 us per 64 positions, the sequential kernel ~0.2 us per
+  // position. The 0.8B forward, sequential against chunked, at 1 sequence of
+  // 128 positions 3.13 / 3.15 ms, 160 3.49 / 3.42, 256 4.28 / 3.91; 2 of 160
+  // 4.27 / 4.05; 4 of 160 6.20 / 5.57; 8 of 224 13.5 / 11.6. At 4 to 32 heads
+  // of 64 or 128, 1 to 4 sequences and 160 to 256 positions the chunked form is
+  // 1 to 45% faster per forward; at 128 it is 1% slower to 29% faster.
   const char *ch_env = std::getenv("RXW8_Q35_CHUNKED");
   const int ch_mode = ch_env && ch_env[0] ? (ch_env[0] == '1' ? 1 : 0) : -1;
-  const bool chunked = m->chunk_ws && (ch_mode == 1 || (ch_mode < 0 && (S >= 256 || (B == 1 && S >= 160))));
+  const bool chunked = m->chunk_ws && (ch_mode == 1 || (ch_mode < 0 && S >= 160));
   Q35MixPrepArgs mp{m->raw, m->f32(L.conv), m->f32(L.a_log), m->f32(L.dt_bias), m->mixed, m->beta,
                     m->g, chunked ? m->lg : nullptr, L.n_in, (int)S, (int)m->Hl, (int)m->Dl,
                     (int)m->cfg.conv_kernel, 1.0f / sqrtf((float)m->Dl), m->f32c ? 1 : 0};

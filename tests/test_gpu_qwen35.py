@@ -133,7 +133,7 @@ def test_chunked_delta_rule(rt, monkeypatch, name, b, s):
     rxw8_q35_delta_scan_d*: per chunk (I + A) Delta = diag(beta) (V -
     diag(Gamma) K S0) solved in parallel, the state carried from chunk to
     chunk on the matrix cores), forced on at every length here (the default
-    takes it from 256 positions), against the sequential recurrence forced on:
+    takes it from 160 positions), against the sequential recurrence forced on:
     one partial chunk, exactly one chunk, several with a partial last one, Dl
     64 and 128; both within TOL of the oracle and within 1e-4 of each other
     (the same terms, reassociated)."""
@@ -151,6 +151,23 @@ def test_chunked_delta_rule(rt, monkeypatch, name, b, s):
           f"between {e_pair:.2e}")
     assert e_c <= TOL and e_s <= TOL
     assert e_pair <= 1e-4
+
+
+@pytest.mark.parametrize("b,s,chunked", [(1, 159, False), (2, 159, False), (1, 160, True), (2, 160, True),
+                                         (2, 255, True)])
+def test_default_delta_rule(rt, monkeypatch, b, s, chunked):
+    """The default takes the chunked form from 160 positions, whatever the
+    batch: its bits are those of the one form, and not those of the other."""
+    cfg = dict(CONFIGS["mid"], layers=[q35.LINEAR], max_seq=256)
+    p = q35.random_params(cfg, seed=65, std=0.05)
+    ids = np.random.default_rng(66).integers(0, cfg["vocab"], (b, s))
+    default = run(rt, build(rt, cfg, p), ids)
+    forced = []
+    for mode in ("0", "1"):
+        monkeypatch.setenv("RXW8_Q35_CHUNKED", mode)
+        forced.append(run(rt, build(rt, cfg, p), ids))
+    assert not np.array_equal(*forced)
+    np.testing.assert_array_equal(default, forced[chunked])
 
 
 @pytest.mark.parametrize("s", [4090, 4160, 4200, 5000, 8200])
