@@ -25,7 +25,9 @@
 // for one wave per row on the VALU; causal prefill of 7 x 425 rows, 32 / 4
 // heads, D = 256: 245 us (85 TFLOP/s) against 9.7 ms. What is left between
 // that and the rate is the softmax and copy issue, which overlap the other
-// waves' MFMAs only in part (MFMA pipes 39-55% busy).
+// waves' MFMAs only in part; under the causal mask (MFMA pipes 21% busy) also
+// the round of workgroups, which lasts as long as the row tile that sees every
+// key.
 // A tile whose mask entries are all -inf for a wave's rows adds exactly nothing
 // when its K and V values are ordinary numbers; the wave then skips its
 // products (after a look at the tile in LDS: NaN and infinities still reach the
