@@ -1087,9 +1087,9 @@ __device__ void delta_chunk(const Q35ChunkArgs &a) {
 // 16 (w - 4) .. + 15 beside them. The state and Delta pass between waves
 // through LDS, columns major (16-byte reads and writes), two barriers a chunk.
 // The serial chain bounds it (64 MFMAs and the two exchanges per 64 positions;
-// the matrix cores of the CUs that it runs on are busy 37% of it). At 500 positions, 16 heads of 128: 38.7
-// -> 33 us against four waves doing both parts with three barriers and 4-byte
-// exchanges.
+// the matrix cores of the CUs that it runs on are busy 37% of it). At 500
+// positions, 16 heads of 128: 38.7 -> 33 us against four waves doing both parts
+// with three barriers and 4-byte exchanges.
 template <int DL>
 __device__ void delta_scan(const Q35ChunkArgs &a) {
   constexpr int C = 64, KQ = DL / 4, GROUPS = DL / 16, IT = DL / 64;
