@@ -55,3 +55,21 @@ def test_rings_and_late_maxima(rt, group, rows, starts, scale, q_bf16):
     ref = reference(q, kc, vc, starts, 128 ** -0.5 if scale is None else scale)
     assert np.isfinite(out).all()
     assert rel_err(out, ref) <= TOL
+
+
+@pytest.mark.parametrize("group", [1, 2, 4, 8])
+@pytest.mark.parametrize("rows,start", [(1, 0), (1, 63), (17, 40), (64, 0), (64, 1), (65, 0)])
+@pytest.mark.parametrize("q_bf16", [True, False])
+def test_one_and_two_blocks(rt, group, rows, start, q_bf16):
+    """A single block of 64 keys runs both heads of a workgroup in step, two
+    run them half a step apart."""
+    import rxla_amd as r
+    rng = np.random.default_rng(64 * rows + start + group)
+    q, kc, vc = make(rng, 2, rows, 2 * group, 2, 130)
+    if q_bf16:
+        q = oracle.round_bf16(q)
+    qb = rt.buffer(oracle.bf16_bits(q), r.DType.BF16) if q_bf16 else rt.buffer(q)
+    starts = np.array([start, max(0, start - 3)], np.int32)
+    out = r.grouped_query_attention_prefill(rt, qb, rt.buffer(kc, r.DType.BF16), rt.buffer(vc, r.DType.BF16),
+                                            rt.buffer(starts), out_dtype=r.DType.F32).to_numpy()
+    assert rel_err(out, reference(q, kc, vc, starts, 128 ** -0.5)) <= TOL
