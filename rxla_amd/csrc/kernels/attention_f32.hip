@@ -471,6 +471,19 @@ __device__ void gqa_tile(const GqaTileArgs &a) {
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * (OPS + 4)) : "memory");
     else
       asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * OPS) : "memory");
+    // V rows past the last key repeat it, with weight 0, which would make NaN of
+    // an infinity: each wave puts zeros over those that it has copied
+    if (t < t1 && 16 * t + 16 > nkeys) {
+      int at = lane;
+      unsigned z = 0;
+      asm volatile("" : "+v"(at), "+v"(z));  // (formed here: kept through the loop they cost D = 256 registers)
+#pragma unroll
+      for (int x = 0; x < OPS; ++x) {
+        const int in = x * RG + rg;
+        if (in >= NI && 16 * t + krow[x] >= nkeys)
+          *(u32x4 *)(ring + bsel * 2 * TILEB + in * 1024 + 16 * at) = u32x4{z, z, z, z};
+      }
+    }
     __syncthreads();
     issue(n + NB - 1);  // into the buffer read before this barrier
     bool work = t < t1 && 16 * t < vis_max;  // wave-uniform
@@ -528,12 +541,11 @@ __device__ void gqa_tile(const GqaTileArgs &a) {
         p[c] = 16 * t + 4 * j + c < row.vis ? s : kNegInf;
       }
       softmax_step<D>(st, p);
-      // a key that some row of the wave must not see (one past a causal row's,
-      // or the last key again in the rows a tile has past it) may hold
+      // a key that some row of the wave must not see (causal starts) may hold
       // anything: a product 0 x NaN or 0 x inf would reach that row, so such a
       // tile's products are formed per row and key
       bool plain = true;
-      if (16 * t + 16 > vis_min) plain = below<BF, TILEB>(vt, lane, kInfBits);
+      if (16 * t + 16 > vis_min && vis_min < nkeys) plain = below<BF, TILEB>(vt, lane, kInfBits);
       if (plain) {
         if constexpr (!PRE) read_v(0), read_v(1);
         if constexpr (D == 256) read_v(2), read_v(3);
@@ -679,10 +691,13 @@ __device__ void gqa_quad(const GqaTileArgs &a) {
   const int NBH = a.NB * a.Hkv, G = a.Hq / a.Hkv, R = G * a.Sq;
   const int bh = blockIdx.x % NBH, split = blockIdx.x / NBH;
   const int b = bh / a.Hkv, kvh = bh - b * a.Hkv;
-  const int slot = a.slots ? a.slots[b] : b;
+  const int slot = __builtin_amdgcn_readfirstlane(a.slots ? a.slots[b] : b);
   const char *kp = (const char *)a.k + (slot * a.k_sb + kvh * a.k_sh) * ES;
   const char *vp = (const char *)a.v + (slot * a.v_sb + kvh * a.v_sh) * ES;
-  const int nkeys = row_vis(a, b, a.Sq - 1), vis_min = row_vis(a, b, 0);
+  const int nkeys = __builtin_amdgcn_readfirstlane(row_vis(a, b, a.Sq - 1)), vis_min = row_vis(a, b, 0);
+  // (V rows past the last key read as zeros: weight 0 times what that key holds
+  // would be NaN for an infinity)
+  const __amdgpu_buffer_rsrc_t v_rsrc = buf_rsrc(vp, (uint32_t)nkeys * ROWB);
   const int ntiles = (nkeys + 15) / 16, per = (ntiles + a.nsplit - 1) / a.nsplit;
   const int t0 = split * per, t1 = min(ntiles, t0 + per);
   KPiece kf[4][NK];
@@ -699,7 +714,8 @@ __device__ void gqa_quad(const GqaTileArgs &a) {
   auto load_v = [&](int t) {
 #pragma unroll
     for (int x = 0; x < BPG; ++x)
-      vf[x] = *(const typename T::Piece *)(vp + (uint32_t)min(16 * t + grp * BPG + x, nkeys - 1) * ROWB + 16 * vcol);
+      vf[x] = __builtin_bit_cast(typename T::Piece, __builtin_amdgcn_raw_buffer_load_b128(
+                                                        v_rsrc, (uint32_t)(16 * t + grp * BPG + x) * ROWB + 16 * vcol, 0, 0));
   };
   const int tb = t0 + wv;
   if (tb < t1) {
@@ -783,7 +799,7 @@ __device__ void gqa_quad(const GqaTileArgs &a) {
       l[s] += p[s];
     }
     bool plain = true;
-    if (16 * t + 16 > vis_min) {  // keys that some row must not see (see gqa_tile)
+    if (16 * t + 16 > vis_min && vis_min < nkeys) {  // keys that some row must not see (see gqa_tile)
       // (on the raw bits: sharing the widened values with the products would
       // keep them all in registers)
       uint32_t hi = 0, lo = 0;
