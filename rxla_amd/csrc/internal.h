@@ -107,6 +107,7 @@ struct Runtime {
   std::string name;
   hipStream_t own_stream = nullptr;
   hipStream_t stream = nullptr;
+  bool own_stream_known = false;  // a caller has asked for its handle, and so may capture it
   std::vector<hipModule_t> modules;
   std::unordered_map<std::string, hipFunction_t> functions;
   std::recursive_mutex mu;

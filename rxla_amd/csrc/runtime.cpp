@@ -155,6 +155,8 @@ void rt_free(Runtime *rt, void *ptr, size_t bytes) {
 }
 
 bool stream_capturing(const Runtime *rt) {
+  // (asking HIP costs 0.13 us of a 6.6 us call)
+  if (rt->stream == rt->own_stream && !rt->own_stream_known) return rt->plan_capture;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(rt->stream, &cs) != hipSuccess) {
     (void)hipGetLastError();
@@ -405,6 +407,8 @@ int rxw8_runtime_set_stream(rxw8_runtime *rt, void *hip_stream) {
 
 int rxw8_runtime_stream(rxw8_runtime *rt, void **hip_stream) {
   if (!rt || !hip_stream) return fail(RXW8_INVALID_ARGUMENT, "NULL argument");
+  std::lock_guard<std::recursive_mutex> g(rt->mu);
+  rt->own_stream_known |= rt->stream == rt->own_stream;
   *hip_stream = (void *)rt->stream;
   return RXW8_OK;
 }

@@ -67,18 +67,20 @@ LINEARS = {  # kind: (rows, n, k, x, compute), a larger call of the same runtime
 }
 
 
+@pytest.mark.parametrize("given", [True, False])
 @pytest.mark.parametrize("kind", list(LINEARS))
-def test_a_captured_call_outlives_its_workspaces(monkeypatch, kind):
-    """A caller's graph holds the addresses of the workspaces that its calls
-    used. A larger eager call replaces them; the replays still give the eager
-    result and touch nothing that was allocated since."""
+def test_a_captured_call_outlives_its_workspaces(monkeypatch, kind, given):
+    """A caller's graph (of a stream that it gave the runtime, or of the
+    runtime's own) holds the addresses of the workspaces that its calls used. A
+    larger eager call replaces them; the replays still give the eager result
+    and touch nothing that was allocated since."""
     import torch
     import rxla_amd as rx
 
     small, large, ks = LINEARS[kind]
     monkeypatch.setenv("RXW8_MID_KS", ks)
     own = rx.Runtime(0)
-    stream = torch.cuda.Stream()
+    stream = torch.cuda.Stream() if given else torch.cuda.ExternalStream(own.stream())
     g = torch.Generator(device="cuda").manual_seed(5)
     rand = lambda *s: torch.randn(*s, generator=g, device="cuda")  # noqa: E731
     keep = []
