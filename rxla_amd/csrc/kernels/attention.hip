@@ -1148,9 +1148,9 @@ struct No { static constexpr bool value = false; };
 // copies in rings of 4 blocks, a bf16 q without a lo part (the scale goes to
 // the scores instead: two thirds of the matrix work), no row maximum unless
 // the reference moves, waves past the last row idle: 4 x 777 rows at 500 on,
-// 32 heads, 91 -> 62 us; 4 x 2048 rows 220 -> 170. What bounds it now: the
-// LDS reads of a matrix half, 32 KiB a wave beside its MFMAs (matrix cores 37%
-// busy at 8 x 1024 rows, 16 / 8 heads, f32 q: 62 us).
+// 32 heads, 91 -> 60 us; 4 x 2048 rows 220 -> 170. What bounds it now: the
+// LDS reads of a matrix half, 32 KiB a wave beside its MFMAs (matrix cores 38%
+// busy at 8 x 1024 rows, 16 / 8 heads, f32 q: 59.8 us).
 template <int G, int R, bool LO>
 __device__ void attn_prefill_rt(const PrefillArgs &a) {
   extern __shared__ __attribute__((aligned(16))) uint16_t pf_lds[];  // [NB][K block] [NB][V block]
